@@ -5,17 +5,30 @@
 //   q, k = rotary_emb(positions, q, k)           rotary_embedding.py:6-17, 37-55
 // With no norm weights it is the rotary embedding alone (Qwen2, qwen2.py:91-92).
 //
-// One (token, head) row per 16 lanes, 4 rows per wavefront.  Lane j of a row
-// holds E = D/32 consecutive elements of each half of the head dimension,
-// [E j, E j + E) and [D/2 + E j, ...), so the rotation pairs (i, i + D/2) are
-// lane-local and only the sum of squares crosses lanes (4 xor shuffles).
+// A wave takes kChunks x 64/LPR head rows of one token, LPR = D/16 lanes per row.
+// Lane j of a row holds 8 consecutive elements of each half of the head dimension,
+// [8 j, 8 j + 8) and [D/2 + 8 j, ...), so the rotation pairs (i, i + D/2) are
+// lane-local and only the sum of squares crosses lanes (xor shuffles over LPR
+// lanes).
+//
+// What bounds it: HBM (each row is read once and written once).  So a lane moves 16
+// bytes per access and issues all its rows' loads before any of them is used (4 KiB in
+// flight per wave at D = 128), the token's cos/sin row is loaded once for all of a
+// wave's heads (per head it is twice the bytes of the row itself, through L1), and no
+// index needs a division.  Stores are non-temporal.  8813 tokens, heads 32/8, D = 128 (185 MB):
+// 46.4 us with 8-byte accesses, one row per lane group and cos/sin per head; 40.5 us in
+// this form with 3 chunks per wave, 39.9 with 2, 42.2 with 1, 46.4 with 5; with the
+// non-temporal stores 35.2 us = 5.26 TB/s (a 2 GiB device copy: 4.9 TB/s).  With the
+// attention that reads q and k right after: a prefill of those tokens 269.5 -> 270.9 us,
+// a decode of 128 rows 34.3 -> 34.0 us (producer and attention together, plain against
+// non-temporal).
 //
 // Arithmetic follows the reference's eager op sequence, rounding where it
 // rounds: fp32 x, mean of squares, x * rsqrt(mean + eps) rounded to bf16, times
 // the bf16 weight rounded to bf16; then fp32 x1*cos - x2*sin and x2*cos + x1*sin
 // with every product and sum rounded separately (no FMA contraction), rounded
 // to bf16.  The sum of squares runs in this kernel's order (a lane's squares,
-// then a 16-lane butterfly), which can move the mean by an fp32 ulp against
+// then a butterfly over the row's lanes), which can move the mean by an fp32 ulp against
 // torch's reduction and so, rarely, an output by one bf16 ulp.  Memory-bound:
 // each row is read once and written once; the cos/sin row of a token is shared
 // by its heads through the caches.
@@ -26,125 +39,180 @@ namespace nva {
 
 namespace {
 
-template <int E>
-struct Half;
-template <>
-struct Half<4> {  // head_dim 128: 4 bf16 = 8 bytes per half
-  typedef u32x2 T;
-  __device__ static T load(const uint16_t* p) { return ld8(p); }
-  __device__ static void store(uint16_t* p, T v) { *reinterpret_cast<u32x2*>(p) = v; }
-  __device__ static uint32_t word(const T& v, int i) { return v[i]; }
-  __device__ static void set(T& v, int i, uint32_t w) { v[i] = w; }
-};
-template <>
-struct Half<2> {  // head_dim 64: 2 bf16 = 4 bytes per half
-  typedef uint32_t T;
-  __device__ static T load(const uint16_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
-  __device__ static void store(uint16_t* p, T v) { *reinterpret_cast<uint32_t*>(p) = v; }
-  __device__ static uint32_t word(const T& v, int) { return v; }
-  __device__ static void set(T& v, int, uint32_t w) { v = w; }
-};
+constexpr int kChunks = 2;         // head chunks of a token that one wave takes
+constexpr int kTokensPerGroup = 4;  // waves per workgroup, one token each
+constexpr int64_t kMaxGroups = int64_t{1} << 22;  // tokens beyond 4 per workgroup: further rounds of the grid
 
-__device__ __forceinline__ float bf16_round(float x) {
-  return bf16_bits_to_f32(pack_bf16x2(x, 0.f) & 0xffffu);
+// 8 bf16 of a row: one 16-byte access, or four of 4 bytes where a pointer or a row
+// stride does not allow it.
+template <bool WIDE>
+__device__ __forceinline__ u32x4 load8(const uint16_t* p) {
+  if constexpr (WIDE) return ld16(p);
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(p);
+  return u32x4{w[0], w[1], w[2], w[3]};
+}
+template <bool WIDE>
+__device__ __forceinline__ void store8(uint16_t* p, u32x4 v) {
+  if constexpr (WIDE) {
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+  } else {
+    uint32_t* w = reinterpret_cast<uint32_t*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = v[i];
+  }
+}
+template <bool WIDE>
+__device__ __forceinline__ void load8f(const float* p, float (&f)[8]) {
+  if constexpr (WIDE) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f[i] = a[i];
+      f[4 + i] = b[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = p[i];
+  }
 }
 
-__device__ __forceinline__ float sum16(float v) {
-  // xor butterflies within each 16-lane row group
+__device__ __forceinline__ void unpack8(u32x4 w, float (&f)[8]) {
 #pragma unroll
-  for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, 16);
-  return v;
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = bf16_bits_to_f32(w[i] & 0xffffu);
+    f[2 * i + 1] = __builtin_bit_cast(float, w[i] & 0xffff0000u);
+  }
+}
+
+// Round 8 values to bf16.
+__device__ __forceinline__ void round8(float (&f)[8]) {
+  u32x4 w;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(f[2 * i], f[2 * i + 1]);
+  unpack8(w, f);
 }
 
 }  // namespace
 
-template <int D>
-__global__ __launch_bounds__(256) void qk_norm_rope_kernel(QKNormRopeParams p) {
+template <int D, bool WIDE>
+__global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNormRopeParams p) {
   // every product and sum rounds on its own, as the reference's separate ops do:
   // no FMA contraction anywhere in this function
 #pragma clang fp contract(off)
-  constexpr int E = D / 32;
-  using H = Half<E>;
+  constexpr int LPR = D / 16;      // lanes per row
+  constexpr int RPW = 64 / LPR;    // rows (heads) per wave and chunk
   const int lane = threadIdx.x & 63;
-  const int j = lane & 15;
-  const int64_t row = (static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 4 + (lane >> 4);
+  const int j = lane & (LPR - 1);
   const int heads = p.num_heads + p.num_kv_heads;
-  const bool valid = row < p.num_tokens * heads;  // no early return: the shuffles need the whole group
-  const int64_t t = valid ? row / heads : 0;
-  const int hh = valid ? static_cast<int>(row - t * heads) : 0;
-  const bool is_q = hh < p.num_heads;
-  const uint16_t* src = is_q ? p.q + t * p.q_row_stride + hh * D
-                             : p.k + t * p.k_row_stride + (hh - p.num_heads) * D;
-  uint16_t* dst = is_q ? p.q_out + t * p.q_out_row_stride + hh * D
-                       : p.k_out + t * p.k_out_row_stride + (hh - p.num_heads) * D;
-
-  typename H::T lo = H::load(src + E * j), hi = H::load(src + D / 2 + E * j);
-  float x1[E], x2[E];
+  const int h0 = static_cast<int>(blockIdx.y) * kChunks * RPW;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kTokensPerGroup;
+  for (int64_t t = static_cast<int64_t>(blockIdx.x) * kTokensPerGroup +
+                   __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+       t < p.num_tokens; t += step) {
+    int64_t pos = p.positions[t];
+    const uint16_t* src[kChunks];
+    uint16_t* dst[kChunks];
+    u32x4 lo[kChunks], hi[kChunks];
 #pragma unroll
-  for (int w = 0; w < E / 2; ++w) {
-    x1[2 * w] = bf16_bits_to_f32(H::word(lo, w) & 0xffffu);
-    x1[2 * w + 1] = bf16_bits_to_f32(H::word(lo, w) >> 16);
-    x2[2 * w] = bf16_bits_to_f32(H::word(hi, w) & 0xffffu);
-    x2[2 * w + 1] = bf16_bits_to_f32(H::word(hi, w) >> 16);
-  }
-
-  if (p.q_weight) {  // RMSNorm over the head dimension (uniform branch)
-    float ss = 0.f;
+    for (int c = 0; c < kChunks; ++c) {
+      const int hh = h0 + c * RPW + lane / LPR;
+      const bool is_q = hh < p.num_heads;
+      src[c] = is_q ? p.q + t * p.q_row_stride + hh * D : p.k + t * p.k_row_stride + (hh - p.num_heads) * D;
+      dst[c] = is_q ? p.q_out + t * p.q_out_row_stride + hh * D
+                    : p.k_out + t * p.k_out_row_stride + (hh - p.num_heads) * D;
+      lo[c] = hi[c] = u32x4{0u, 0u, 0u, 0u};
+      if (hh < heads) {
+        lo[c] = load8<WIDE>(src[c] + 8 * j);
+        hi[c] = load8<WIDE>(src[c] + D / 2 + 8 * j);
+      }
+    }
+    // cache row = [cos(D/2) | sin(D/2)] of the clamped position
+    pos = pos < 0 ? 0 : (pos >= p.max_position ? p.max_position - 1 : pos);
+    float cs[8], sn[8];
+    load8f<WIDE>(p.cos_sin + pos * D + 8 * j, cs);
+    load8f<WIDE>(p.cos_sin + pos * D + D / 2 + 8 * j, sn);
 #pragma unroll
-    for (int e = 0; e < E; ++e) ss = (ss + x1[e] * x1[e]) + x2[e] * x2[e];
-    ss = sum16(ss);
-    const float r = rsqrtf(ss / static_cast<float>(D) + p.eps);
-    const uint16_t* wt = is_q ? p.q_weight : p.k_weight;
-    typename H::T wl = H::load(wt + E * j), wh = H::load(wt + D / 2 + E * j);
+    for (int c = 0; c < kChunks; ++c) {
+      if (h0 + c * RPW >= heads) break;  // uniform: the whole chunk lies past the last head
+      const int hh = h0 + c * RPW + lane / LPR;
+      float x1[8], x2[8];
+      unpack8(lo[c], x1);
+      unpack8(hi[c], x2);
+      if (p.q_weight) {  // RMSNorm over the head dimension (uniform branch)
+        float ss = 0.f;
 #pragma unroll
-    for (int w = 0; w < E / 2; ++w) {
+        for (int e = 0; e < 8; ++e) ss = (ss + x1[e] * x1[e]) + x2[e] * x2[e];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const float w1 = bf16_bits_to_f32(b ? H::word(wl, w) >> 16 : H::word(wl, w) & 0xffffu);
-        const float w2 = bf16_bits_to_f32(b ? H::word(wh, w) >> 16 : H::word(wh, w) & 0xffffu);
-        x1[2 * w + b] = bf16_round(bf16_round(x1[2 * w + b] * r) * w1);
-        x2[2 * w + b] = bf16_round(bf16_round(x2[2 * w + b] * r) * w2);
+        for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, LPR);
+        const float r = rsqrtf(ss / static_cast<float>(D) + p.eps);
+        const uint16_t* wt = hh < p.num_heads ? p.q_weight : p.k_weight;
+        float w1[8], w2[8];
+        unpack8(load8<WIDE>(wt + 8 * j), w1);
+        unpack8(load8<WIDE>(wt + D / 2 + 8 * j), w2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          x1[e] *= r;
+          x2[e] *= r;
+        }
+        round8(x1);
+        round8(x2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          x1[e] *= w1[e];
+          x2[e] *= w2[e];
+        }
+        round8(x1);
+        round8(x2);
+      }
+      u32x4 o1, o2;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        float y1[2], y2[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int e = 2 * w + b;
+          y1[b] = x1[e] * cs[e] - x2[e] * sn[e];
+          y2[b] = x2[e] * cs[e] + x1[e] * sn[e];
+        }
+        o1[w] = pack_bf16x2(y1[0], y1[1]);
+        o2[w] = pack_bf16x2(y2[0], y2[1]);
+      }
+      if (hh < heads) {
+        store8<WIDE>(dst[c] + 8 * j, o1);
+        store8<WIDE>(dst[c] + D / 2 + 8 * j, o2);
       }
     }
   }
+}
 
-  // rotary embedding: cache row = [cos(D/2) | sin(D/2)] of the clamped position
-  int64_t pos = valid ? p.positions[t] : 0;
-  pos = pos < 0 ? 0 : (pos >= p.max_position ? p.max_position - 1 : pos);
-  const float* cs = p.cos_sin + pos * D;
-  float c[E], s[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    c[e] = cs[E * j + e];
-    s[e] = cs[D / 2 + E * j + e];
-  }
-  typename H::T o1, o2;
-#pragma unroll
-  for (int w = 0; w < E / 2; ++w) {
-    float y1[2], y2[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int e = 2 * w + b;
-      y1[b] = x1[e] * c[e] - x2[e] * s[e];
-      y2[b] = x2[e] * c[e] + x1[e] * s[e];
-    }
-    H::set(o1, w, pack_bf16x2(y1[0], y1[1]));
-    H::set(o2, w, pack_bf16x2(y2[0], y2[1]));
-  }
-  if (valid) {
-    H::store(dst + E * j, o1);
-    H::store(dst + D / 2 + E * j, o2);
-  }
+// The wide accesses need 16-byte aligned rows, weights and table (rows of every engine
+// tensor are); other inputs take 4-byte accesses of the same kernel.
+static bool rows_aligned16(const QKNormRopeParams& p) {
+  auto a = [](const void* x) { return reinterpret_cast<uintptr_t>(x) % 16 == 0; };
+  return a(p.q) && a(p.k) && a(p.q_out) && a(p.k_out) && a(p.q_weight) && a(p.k_weight) && a(p.cos_sin) &&
+         (p.q_row_stride | p.k_row_stride | p.q_out_row_stride | p.k_out_row_stride) % 8 == 0;
 }
 
 hipError_t launch_qk_norm_rope(const QKNormRopeParams& p, hipStream_t stream) {
-  const int64_t rows = p.num_tokens * (p.num_heads + p.num_kv_heads);
-  if (rows <= 0) return hipSuccess;
-  const int64_t blocks = (rows + 15) / 16;  // 4 wavefronts x 4 rows
-  if (p.head_dim == 128)
-    hipLaunchKernelGGL(qk_norm_rope_kernel<128>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL(qk_norm_rope_kernel<64>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
+  const int heads = p.num_heads + p.num_kv_heads;
+  if (p.num_tokens <= 0 || heads <= 0) return hipSuccess;
+  const int per_wave = kChunks * 64 / (p.head_dim / 16);  // heads
+  const int64_t groups = (p.num_tokens + kTokensPerGroup - 1) / kTokensPerGroup;
+  const dim3 grid(static_cast<unsigned>(groups < kMaxGroups ? groups : kMaxGroups),
+                  static_cast<unsigned>((heads + per_wave - 1) / per_wave));
+  const dim3 block(64 * kTokensPerGroup);
+  const bool wide = rows_aligned16(p);
+  if (p.head_dim == 128) {
+    if (wide)
+      hipLaunchKernelGGL((qk_norm_rope_kernel<128, true>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((qk_norm_rope_kernel<128, false>), grid, block, 0, stream, p);
+  } else {
+    if (wide)
+      hipLaunchKernelGGL((qk_norm_rope_kernel<64, true>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((qk_norm_rope_kernel<64, false>), grid, block, 0, stream, p);
+  }
   return hipGetLastError();
 }
 

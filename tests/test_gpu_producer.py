@@ -134,6 +134,30 @@ def test_token_counts_and_positions(dev):
     _assert_close(q, rq, "edge positions", xhat=_normed(case)[0])
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(15, 1, 128), (16, 1, 128), (17, 3, 128), (31, 1, 64), (33, 1, 64)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_head_chunks_and_narrow_rows(dev, nh, nkv, d, norm):
+    """Head counts around a wave's rows (16 heads at d=128, 32 at d=64), and rows that allow only
+    narrow accesses (8 bytes at d=128, 4 at d=64): bit-identical to 16-byte aligned ones."""
+    from nanovllm_amd import workloads as W
+    from nanovllm_amd.layers.qk_norm_rope import qk_norm_rope
+    case = W.make_producer_case(9, nh, nkv, head_dim=d, seed=nh + d, norm=norm, device=dev)
+    q, k = _run(case)
+    rq, rk = _oracle(case)
+    xq, xk = _normed(case)
+    _assert_close(q, rq, "q", exact=not norm, xhat=xq)
+    _assert_close(k, rk, "k", exact=not norm, xhat=xk)
+    off = 4 if d == 128 else 2  # elements
+    width = case.qkv.shape[1]
+    buf = torch.zeros(9, width + 2 * off, dtype=torch.bfloat16, device=dev)
+    buf[:, off:off + width] = case.qkv
+    qn, kn = buf[:, off:off + nh * d], buf[:, off + nh * d:off + (nh + nkv) * d]
+    assert qn.data_ptr() % 16 != 0
+    q2, k2 = qk_norm_rope(case.positions, qn, kn, case.cos_sin_cache, nh, nkv, d, case.q_norm_weight,
+                          case.k_norm_weight, case.eps)
+    assert torch.equal(q2.view(-1), q.view(-1)) and torch.equal(k2.view(-1), k.view(-1))
+
+
 def test_out_of_range_positions_are_clamped(dev):
     from nanovllm_amd import workloads as W
     case = W.make_producer_case(3, 16, 8, max_position=64, positions=[-5, 64, 1000], seed=4, device=dev)
