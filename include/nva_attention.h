@@ -270,6 +270,24 @@ int nva_qk_norm_rope(const void* q, int64_t q_row_stride,
                      const int64_t* positions, int64_t num_tokens,
                      int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, void* stream);
 
+/*
+ * Inputs of a captured decode step: run_model's zero fills and row copies into the graph's
+ * static buffers (model_runner.py:271-280) as one launch.  Rows [0, live_rows) of q_out,
+ * k_out, v_out, slots_out, lens_out and table_out (contiguous, row lengths q_elems, kv_elems
+ * and out_width) take the given rows, table entries from bt_width on 0; rows
+ * [live_rows, rows) become zero rows with slot pad_slot and length 0.  bf16 rows 16-byte
+ * aligned, their lengths and strides a multiple of 8 elements.
+ */
+int nva_stage_decode(const void* q, int64_t q_row_stride,
+                     const void* k, int64_t k_row_stride,
+                     const void* v, int64_t v_row_stride,
+                     const int32_t* slot_mapping, const int32_t* context_lens,
+                     const int32_t* block_table, int64_t bt_row_stride, int32_t bt_width,
+                     int32_t live_rows, int32_t q_elems, int32_t kv_elems,
+                     void* q_out, void* k_out, void* v_out,
+                     int32_t* slots_out, int32_t* lens_out, int32_t* table_out, int32_t out_width,
+                     int32_t rows, int32_t pad_slot, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

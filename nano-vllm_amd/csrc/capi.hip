@@ -562,4 +562,52 @@ int nva_qk_norm_rope(const void* q, int64_t q_row_stride, const void* k, int64_t
   return hip_status(nva::launch_qk_norm_rope(p, static_cast<hipStream_t>(stream)), "qk_norm_rope launch");
 }
 
+int nva_stage_decode(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+                     int64_t v_row_stride, const int32_t* slot_mapping, const int32_t* context_lens,
+                     const int32_t* block_table, int64_t bt_row_stride, int32_t bt_width, int32_t live_rows,
+                     int32_t q_elems, int32_t kv_elems, void* q_out, void* k_out, void* v_out, int32_t* slots_out,
+                     int32_t* lens_out, int32_t* table_out, int32_t out_width, int32_t rows, int32_t pad_slot,
+                     void* stream) {
+  if (live_rows < 0 || rows < live_rows || q_elems <= 0 || kv_elems <= 0 || bt_width < 0 || out_width < bt_width)
+    return fail(NVA_ERR_INVALID_ARGUMENT, "rows must be >= live_rows >= 0, element counts positive, out_width >= bt_width >= 0");
+  if (rows == 0) return ok();
+  if (!q_out || !k_out || !v_out || !slots_out || !lens_out || (out_width > 0 && !table_out) ||
+      (live_rows > 0 && (!q || !k || !v || !slot_mapping || !context_lens || (bt_width > 0 && !block_table))))
+    return fail(NVA_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (live_rows > 0 && (q_row_stride < q_elems || k_row_stride < kv_elems || v_row_stride < kv_elems || bt_row_stride < bt_width))
+    return fail(NVA_ERR_INVALID_ARGUMENT, "row strides must cover their rows");
+  if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(q_out, 16) || !aligned(k_out, 16) ||
+      !aligned(v_out, 16) || (q_elems % 8) || (kv_elems % 8) || (q_row_stride % 8) || (k_row_stride % 8) ||
+      (v_row_stride % 8))
+    return fail(NVA_ERR_UNSUPPORTED, "q/k/v rows must be 16-byte aligned and a multiple of 8 elements");
+  if (!aligned(slot_mapping, 4) || !aligned(context_lens, 4) || !aligned(block_table, 4) || !aligned(slots_out, 4) ||
+      !aligned(lens_out, 4) || !aligned(table_out, 4))
+    return fail(NVA_ERR_INVALID_ARGUMENT, "index tensors must be 4-byte aligned");
+  nva::StageParams p{};
+  p.q = static_cast<const uint16_t*>(q);
+  p.k = static_cast<const uint16_t*>(k);
+  p.v = static_cast<const uint16_t*>(v);
+  p.slots = slot_mapping;
+  p.lens = context_lens;
+  p.table = block_table;
+  p.q_out = static_cast<uint16_t*>(q_out);
+  p.k_out = static_cast<uint16_t*>(k_out);
+  p.v_out = static_cast<uint16_t*>(v_out);
+  p.slots_out = slots_out;
+  p.lens_out = lens_out;
+  p.table_out = table_out;
+  p.q_row_stride = q_row_stride;
+  p.k_row_stride = k_row_stride;
+  p.v_row_stride = v_row_stride;
+  p.table_row_stride = bt_row_stride;
+  p.live = live_rows;
+  p.rows = rows;
+  p.q_elems = q_elems;
+  p.kv_elems = kv_elems;
+  p.width = bt_width;
+  p.out_width = out_width;
+  p.pad_slot = pad_slot;
+  return hip_status(nva::launch_stage_decode(p, static_cast<hipStream_t>(stream)), "stage_decode launch");
+}
+
 }  // extern "C"

@@ -142,6 +142,27 @@ struct GatherParams {
   int32_t head_dim;
 };
 
+// Rows of a captured decode step's static buffers (stage_decode.hip).
+struct StageParams {
+  const uint16_t* q;          // bf16 rows, q_elems each
+  const uint16_t* k;          // bf16 rows, kv_elems each
+  const uint16_t* v;
+  const int32_t* slots;       // [live]
+  const int32_t* lens;        // [live]
+  const int32_t* table;       // [live, >= width]
+  uint16_t* q_out;            // (>= rows, q_elems) contiguous, and so on
+  uint16_t* k_out;
+  uint16_t* v_out;
+  int32_t* slots_out;
+  int32_t* lens_out;
+  int32_t* table_out;         // (>= rows, out_width)
+  int64_t q_row_stride, k_row_stride, v_row_stride, table_row_stride;
+  int32_t live, rows;
+  int32_t q_elems, kv_elems, width, out_width;
+  int32_t pad_slot;
+};
+
+hipError_t launch_stage_decode(const StageParams& p, hipStream_t stream);
 hipError_t launch_store_kvcache(const StoreParams& p, int vec_bytes, hipStream_t stream);
 hipError_t launch_gather_kv(const GatherParams& p, int max_seqlen_k, int kv_dtype, hipStream_t stream);
 hipError_t launch_qk_norm_rope(const QKNormRopeParams& p, hipStream_t stream);

@@ -100,6 +100,15 @@ SIGNATURES = {
         _c_void_p, _i64, _c_void_p, _i64,  # cos_sin_cache, max_position, positions, num_tokens
         _i32, _i32, _i32, _c_void_p,       # num_heads, num_kv_heads, head_dim, stream
     ]),
+    "nva_stage_decode": (_i32, [
+        _c_void_p, _i64, _c_void_p, _i64, _c_void_p, _i64,  # q, q_row_stride, k, k_row_stride, v, v_row_stride
+        _c_void_p, _c_void_p,              # slot_mapping, context_lens
+        _c_void_p, _i64, _i32,             # block_table, bt_row_stride, bt_width
+        _i32, _i32, _i32,                  # live_rows, q_elems, kv_elems
+        _c_void_p, _c_void_p, _c_void_p,   # q_out, k_out, v_out
+        _c_void_p, _c_void_p, _c_void_p, _i32,  # slots_out, lens_out, table_out, out_width
+        _i32, _i32, _c_void_p,             # rows, pad_slot, stream
+    ]),
 }
 
 

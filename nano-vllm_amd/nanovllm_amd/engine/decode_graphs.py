@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _capi
 from ..layers.attention import Attention
 from ..utils.context import reset_context, set_context
 
@@ -101,6 +102,41 @@ class DecodeGraphs:
             reset_context()
         return self
 
+    def _stage(self, size: int, q, k, v, slot_mapping, context_lens, block_tables) -> bool:
+        """The static buffers' rows up to `size` (all that the graph of that size reads)
+        written by one launch (nva_stage_decode).  False, with nothing done, for inputs
+        that the launch does not take as they are -- other types or devices (or another
+        current device), rows that are
+        not contiguous and 16-byte aligned, other shapes -- which the tensor copies of
+        run() convert, or reject."""
+        bs, dev = q.shape[0], self.q.device
+        if bs == 0 or torch.cuda.current_device() != dev.index:
+            return False
+        rows = []
+        for x, buf in ((q, self.q), (k, self.k), (v, self.v)):
+            if x.dtype != torch.bfloat16 or x.device != dev or x.shape[0] != bs or x.numel() != bs * buf.shape[1]:
+                return False
+            if x.dim() == 3:
+                inner = x.stride(2) == 1 and x.stride(1) == x.shape[2]
+            else:
+                inner = x.dim() == 2 and x.stride(1) == 1
+            if not inner or x.stride(0) < buf.shape[1] or x.stride(0) % 8 or x.data_ptr() % 16 or buf.shape[1] % 8:
+                return False
+            rows += [x.data_ptr(), x.stride(0)]
+        for x in (slot_mapping, context_lens):
+            if x.dtype != torch.int32 or x.device != dev or x.shape != (bs,) or not x.is_contiguous():
+                return False
+        bt = block_tables
+        if bt.dtype != torch.int32 or bt.device != dev or bt.dim() != 2 or bt.shape[0] != bs or bt.stride(1) != 1 \
+                or bt.stride(0) < bt.shape[1]:
+            return False
+        _capi.check(_capi.load().nva_stage_decode(
+            *rows, slot_mapping.data_ptr(), context_lens.data_ptr(), bt.data_ptr(), bt.stride(0), bt.shape[1],
+            bs, self.q.shape[1], self.k.shape[1], self.q.data_ptr(), self.k.data_ptr(), self.v.data_ptr(),
+            self.slot_mapping.data_ptr(), self.context_lens.data_ptr(), self.block_tables.data_ptr(),
+            self.max_num_blocks, size, self.pad_slot, torch.cuda.current_stream(dev).cuda_stream))
+        return True
+
     @torch.inference_mode()
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, slot_mapping: torch.Tensor,
             context_lens: torch.Tensor, block_tables: torch.Tensor) -> list[torch.Tensor]:
@@ -117,18 +153,19 @@ class DecodeGraphs:
                 return self._call_layers(q, k, v)
             finally:
                 reset_context()
-        # static buffers: zero, live rows in (model_runner.py:271-280); slots padded with pad_slot
-        self.q.zero_()
-        self.k.zero_()
-        self.v.zero_()
-        self.slot_mapping.fill_(self.pad_slot)
-        self.context_lens.zero_()
-        self.block_tables.zero_()
-        self.q[:bs] = q.reshape(bs, -1)
-        self.k[:bs] = k.reshape(bs, -1)
-        self.v[:bs] = v.reshape(bs, -1)
-        self.slot_mapping[:bs] = slot_mapping
-        self.context_lens[:bs] = context_lens
-        self.block_tables[:bs, : block_tables.shape[1]] = block_tables
+        if not self._stage(size, q, k, v, slot_mapping, context_lens, block_tables):
+            # static buffers: zero, live rows in (model_runner.py:271-280); slots padded with pad_slot
+            self.q.zero_()
+            self.k.zero_()
+            self.v.zero_()
+            self.slot_mapping.fill_(self.pad_slot)
+            self.context_lens.zero_()
+            self.block_tables.zero_()
+            self.q[:bs] = q.reshape(bs, -1)
+            self.k[:bs] = k.reshape(bs, -1)
+            self.v[:bs] = v.reshape(bs, -1)
+            self.slot_mapping[:bs] = slot_mapping
+            self.context_lens[:bs] = context_lens
+            self.block_tables[:bs, : block_tables.shape[1]] = block_tables
         self.graphs[size].replay()
         return [o[:bs] for o in self.layer_outputs[size]]

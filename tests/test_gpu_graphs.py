@@ -171,3 +171,31 @@ def test_fp8_cache_replay_matches_oracle(dev):
                                    v_scale=a.v_scale)
             assert_attn_close(f32(got[li]).reshape(bs, NH, D), decode_reference(case), max_abs=FP8_MAX_ABS,
                               mean_abs=FP8_MAX_ABS, what=f"fp8 graph bs={bs} layer {li} vs oracle")
+
+
+@pytest.mark.parametrize("bs", [1, 5, 16])
+def test_staged_inputs_equal_the_tensor_copies(dev, bs):
+    """The static buffers as the one-launch staging writes them (rows up to the graph's size)
+    equal the fills and copies; inputs it does not take (int64 slots, unaligned or
+    transposed rows) go through the copies with the same replayed result."""
+    from nanovllm_amd.engine.decode_graphs import DecodeGraphs
+    layers = _layers(dev, 1, 64, seed=7)
+    graphs = DecodeGraphs(layers, max_bs=16, max_num_blocks=4).capture()
+    q, k, v, slots, ctx, bt = _batch(dev, bs, 3, 64, seed=bs)
+    size = min(x for x in graphs.graph_bs if x >= bs)
+    for buf in (graphs.q, graphs.k, graphs.v, graphs.slot_mapping, graphs.context_lens, graphs.block_tables):
+        buf.fill_(7)  # what an earlier, larger step left
+    qkv = torch.cat([q, k, v], dim=1)  # strided rows, as the fused projection leaves them
+    D2 = NH * D
+    want = torch.stack(graphs.run(qkv[:, :D2], qkv[:, D2:D2 + NKV * D], qkv[:, D2 + NKV * D:].view(bs, NKV, D), slots,
+                                  ctx, bt)).clone()
+    for buf, rows, fill in ((graphs.q, q, 0), (graphs.k, k, 0), (graphs.v, v, 0), (graphs.slot_mapping, slots, -1),
+                            (graphs.context_lens, ctx, 0)):
+        assert torch.equal(buf[:bs], rows) and bool((buf[bs:size] == fill).all())
+    assert torch.equal(graphs.block_tables[:bs, :3], bt) and not bool(graphs.block_tables[:bs, 3:].any())
+    assert not bool(graphs.block_tables[bs:size].any())
+    odd = torch.empty(bs, D2 + 1, dtype=torch.bfloat16, device=dev)[:, 1:]
+    odd.copy_(q)
+    for args in ((q, k, v, slots.long(), ctx, bt), (odd, k, v, slots, ctx, bt),
+                 (q.t().contiguous().t(), k, v, slots, ctx, bt), (q.float(), k, v, slots, ctx, bt)):
+        assert torch.equal(torch.stack(graphs.run(*args)), want)
