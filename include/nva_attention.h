@@ -118,6 +118,28 @@ int nva_prefill(const void* q, int64_t q_row_stride,
                 void* out, int64_t out_row_stride,
                 void* workspace, int64_t workspace_bytes, void* stream);
 
+/*
+ * One prefill step of Attention.forward without a cached prefix (attention.py:58-73): the store
+ * of the fresh rows (nva_store_kvcache with key = k, value = v) followed by the packed prefill
+ * over them (nva_prefill with block_table NULL), with the results of the two calls.  The
+ * attention reads the fresh rows, not the caches, so over a bf16 cache with 16-byte aligned
+ * rows the store runs inside the prefill launch; otherwise (an fp8 cache, other alignments,
+ * GQA group 1 at head_dim 128, a large launch without a workspace, or q, k, v or out inside a
+ * cache) the store kernel runs first.  num_queries: rows of q and out.
+ */
+int nva_store_prefill(void* k_cache, void* v_cache, int64_t num_slots,
+                      const int32_t* slot_mapping, int64_t num_tokens, int32_t cache_dtype,
+                      const float* k_scale, const float* v_scale,
+                      const void* q, int64_t q_row_stride, int64_t num_queries,
+                      const void* k, int64_t k_row_stride,
+                      const void* v, int64_t v_row_stride,
+                      const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                      int32_t num_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k,
+                      int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                      float softmax_scale,
+                      void* out, int64_t out_row_stride,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Bytes of the optional nva_prefill workspace (a constant of the library). */
 int64_t nva_prefill_workspace_bytes(void);
 

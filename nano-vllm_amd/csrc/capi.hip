@@ -132,13 +132,19 @@ int nva_store_kvcache(const void* key, int64_t key_row_stride, const void* value
   return hip_status(nva::launch_store_kvcache(p, vec, static_cast<hipStream_t>(stream)), "store_kvcache launch");
 }
 
-int nva_prefill(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+}  // extern "C"
+
+namespace {
+
+// nva_prefill's body.  `store`: the store that comes before it (null: none), fused into the
+// launch by launch_prefill where it can be.
+int prefill_impl(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
                 int64_t v_row_stride, const int32_t* block_table, int64_t bt_row_stride,
                 int32_t max_blocks_per_seq, int32_t block_size, int64_t num_blocks,
                 const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int32_t num_seqs,
                 int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads, int32_t num_kv_heads,
                 int32_t head_dim, float softmax_scale, void* out, int64_t out_row_stride, void* workspace,
-                int64_t workspace_bytes, void* stream) {
+                int64_t workspace_bytes, void* stream, const nva::StoreParams* store = nullptr, int store_vec = 0) {
   if (head_dim != 128 && head_dim != 64)
     return fail(NVA_ERR_UNSUPPORTED, "head_dim %d not supported (64 or 128)", head_dim);
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
@@ -146,7 +152,10 @@ int nva_prefill(const void* q, int64_t q_row_stride, const void* k, int64_t k_ro
   if (num_heads > 65535) return fail(NVA_ERR_UNSUPPORTED, "num_heads above 65535");
   if (num_seqs < 0 || max_seqlen_q < 0) return fail(NVA_ERR_INVALID_ARGUMENT, "num_seqs and max_seqlen_q must be >= 0");
   if (num_seqs > 65535) return fail(NVA_ERR_UNSUPPORTED, "num_seqs above 65535");
-  if (num_seqs == 0 || max_seqlen_q == 0) return ok();
+  if (num_seqs == 0 || max_seqlen_q == 0) {
+    if (!store) return ok();
+    return hip_status(nva::launch_store_kvcache(*store, store_vec, static_cast<hipStream_t>(stream)), "store_kvcache launch");
+  }
   if (!q || !k || !v || !out || !cu_seqlens_q || !cu_seqlens_k) return fail(NVA_ERR_INVALID_ARGUMENT, "null pointer argument");
   const int64_t hd = static_cast<int64_t>(num_heads) * head_dim;
   const int64_t kd = static_cast<int64_t>(num_kv_heads) * head_dim;
@@ -208,8 +217,66 @@ int nva_prefill(const void* q, int64_t q_row_stride, const void* k, int64_t k_ro
     p.split_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + nva::kPrefillSplitPartOffset);
     p.split_err = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + nva::kPrefillErrOffset);
   }
-  return hip_status(nva::launch_prefill(p, max_seqlen_q, max_seqlen_k, static_cast<hipStream_t>(stream)),
+  return hip_status(nva::launch_prefill(p, max_seqlen_q, max_seqlen_k, static_cast<hipStream_t>(stream), store,
+                                        store_vec),
                     "prefill launch");
+}
+
+// Whether `rows` rows of `width` elements at `base` (row stride `stride`, bf16) touch the
+// `bytes` bytes at `other`.
+bool rows_overlap(const void* base, int64_t rows, int64_t stride, int64_t width, const void* other, int64_t bytes) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(base), c = reinterpret_cast<uintptr_t>(other);
+  const uintptr_t a_end = a + static_cast<uintptr_t>((rows - 1) * stride + width) * 2;
+  return rows > 0 && a < c + static_cast<uintptr_t>(bytes) && c < a_end;
+}
+
+}  // namespace
+
+extern "C" {
+
+int nva_prefill(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
+                int64_t v_row_stride, const int32_t* block_table, int64_t bt_row_stride,
+                int32_t max_blocks_per_seq, int32_t block_size, int64_t num_blocks,
+                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int32_t num_seqs,
+                int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads, int32_t num_kv_heads,
+                int32_t head_dim, float softmax_scale, void* out, int64_t out_row_stride, void* workspace,
+                int64_t workspace_bytes, void* stream) {
+  return prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, block_table, bt_row_stride, max_blocks_per_seq,
+                      block_size, num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q, max_seqlen_k,
+                      num_heads, num_kv_heads, head_dim, softmax_scale, out, out_row_stride, workspace,
+                      workspace_bytes, stream);
+}
+
+int nva_store_prefill(void* k_cache, void* v_cache, int64_t num_slots, const int32_t* slot_mapping, int64_t num_tokens,
+                      int32_t cache_dtype, const float* k_scale, const float* v_scale, const void* q,
+                      int64_t q_row_stride, int64_t num_queries, const void* k, int64_t k_row_stride, const void* v,
+                      int64_t v_row_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int32_t num_seqs,
+                      int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads, int32_t num_kv_heads,
+                      int32_t head_dim, float softmax_scale, void* out, int64_t out_row_stride, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  nva::StoreParams sp{};
+  int vec = 2;
+  const int rc = store_setup(k, k_row_stride, v, v_row_stride, k_cache, v_cache, num_slots, slot_mapping, num_tokens,
+                             num_kv_heads, head_dim, cache_dtype, k_scale, v_scale, sp, vec);
+  if (rc != NVA_OK) return rc;
+  bool apart = num_tokens == 0;
+  if (num_tokens > 0) {
+    // Tensors of the attention inside the caches: the store has to be done before it.
+    const int64_t D = static_cast<int64_t>(num_kv_heads) * head_dim, qd = static_cast<int64_t>(num_heads) * head_dim;
+    const int64_t bytes = num_slots * D * (cache_dtype == NVA_DTYPE_BF16 ? 2 : 1);
+    for (const void* c : {k_cache, v_cache})
+      apart = apart || rows_overlap(k, num_tokens, k_row_stride, D, c, bytes) ||
+              rows_overlap(v, num_tokens, v_row_stride, D, c, bytes) ||
+              rows_overlap(q, num_queries, q_row_stride, qd, c, bytes) ||
+              rows_overlap(out, num_queries, out_row_stride, qd, c, bytes);
+    if (apart) {
+      const hipError_t e = nva::launch_store_kvcache(sp, vec, static_cast<hipStream_t>(stream));
+      if (e != hipSuccess) return hip_status(e, "store_kvcache launch");
+    }
+  }
+  return prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, nullptr, 0, 0, 0, 0, cu_seqlens_q,
+                      cu_seqlens_k, num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim,
+                      softmax_scale, out, out_row_stride, workspace, workspace_bytes, stream, apart ? nullptr : &sp, vec);
 }
 
 int64_t nva_prefill_workspace_bytes(void) { return nva::kPrefillWorkspaceBytes; }

@@ -103,6 +103,14 @@ struct PrefillParams {
   // only by the host; split_err[1]: the merge wait's poll limit (0: the
   // default bound, n > 0: n - 1 polls), written by the host.
   uint32_t* split_err;
+  // Store of the fresh rows fused into the launch (packed k/v only; st_rows 0: none):
+  // rows [0, st_rows) of k and v go to cache rows slot_mapping[row] of k_cache and
+  // v_cache (bf16, num_slots rows), slots outside the caches skipped.
+  uint16_t* k_cache;
+  uint16_t* v_cache;
+  const int32_t* slot_mapping;
+  int64_t num_slots;
+  int64_t st_rows;
 };
 
 struct QKNormRopeParams {
@@ -167,7 +175,10 @@ hipError_t launch_store_kvcache(const StoreParams& p, int vec_bytes, hipStream_t
 hipError_t launch_gather_kv(const GatherParams& p, int max_seqlen_k, int kv_dtype, hipStream_t stream);
 hipError_t launch_qk_norm_rope(const QKNormRopeParams& p, hipStream_t stream);
 hipError_t launch_decode(const DecodeParams& p, int kv_dtype, hipStream_t stream);
-hipError_t launch_prefill(const PrefillParams& p, int max_seqlen_q, int max_seqlen_k, hipStream_t stream);
+// `store`: the store of the same call (null: none), fused into the prefill launch where
+// that is possible, launched before it otherwise.
+hipError_t launch_prefill(const PrefillParams& p, int max_seqlen_q, int max_seqlen_k, hipStream_t stream,
+                          const StoreParams* store = nullptr, int store_vec = 0);
 int prefill_positions_per_tile(int group);  // query positions one prefill workgroup covers
 constexpr int kPrefillMaxGroup = 256;        // rows per prefill workgroup bound the GQA group
 // Work queue of the persistent prefill grid: one claim counter per XCD lane,

@@ -201,6 +201,8 @@ struct ItemDesc {
   int ntiles;  // 64-key tiles spanning [0, kmax)
   int split_slot;  // >= 0: one key half of a split item (workspace slot); -1: a whole item
   int bt_off;      // paged: block-table entries before the item's first key (a second key half)
+  int st_row;      // rows of k and v whose store this item carries: from st_row on,
+  int st_n;        // st_n of them
   bool valid;  // false: no item (s < 0) or a tile past the sequence's end
 };
 
@@ -224,6 +226,8 @@ __device__ __forceinline__ ItemDesc item_desc(const PrefillParams& p, const int*
   const int last_pos = min(d.i0 + p.positions_per_tile, d.Lq) - 1;
   d.kmax = max(0, min(d.Lk, last_pos + (d.Lk - d.Lq) + 1));
   d.ntiles = (d.kmax + kBK - 1) / kBK;
+  d.st_row = d.q_start + d.i0;
+  d.st_n = last_pos + 1 - d.i0;
   return d;
 }
 
@@ -373,6 +377,7 @@ __device__ __forceinline__ void key_half(const PrefillParams& p, ItemDesc& d, in
   d.k_start += k0;
   d.Lk -= k0;
   d.split_slot = slot;
+  if (!half) d.st_n = 0;  // the second half holds the item's own positions
 }
 
 // Bound on the merging workgroup's wait for the other half's partial.  With
@@ -567,6 +572,102 @@ __device__ __forceinline__ void item_fetch_tiles(const PrefillParams& p, char* s
     if (t < it.ntiles) st.copy(p, it, smem_all + t * Geom<D>::kTileBytes, PAGED ? page_of(p, st.bt, st.mb, t * kBK) : 0, t);
 }
 
+// The store fused into a packed prefill: every item also writes the cache rows of its
+// own positions (its kv head's K and V).  The attention of such a launch reads the fresh
+// rows, never the caches, so the order of the two does not matter.  Those rows are the
+// last keys of the item, and when its loop ends the ring still holds them: they go from
+// LDS to the caches, with no load but the slots (fetched like the next item's Q).  What
+// it saves is the store launch before the prefill; Attention.forward as a whole, two
+// launches against one: one 16001-token prompt, heads 16/8, 928 -> 910 us; 12 prompts of
+// 100-1024 tokens, heads 14/2, d = 64, 25.3 -> 24.0 us; 8 such prompts, heads 16/8,
+// 30.7 -> 30.2 us (there the separate store had also brought the keys into the L2s).
+// Loading the rows again with the item's first tiles, in place of reading them from the
+// ring, cost the last of these 31.1 us: every workgroup's start is bound by its loads.
+constexpr int kMaxRingRows = 193;  // rows always inside the last kStages tiles, wherever they start
+
+// Pieces of 16 bytes of one row's K and V (one kv head).
+template <int D>
+constexpr int kRowPieces = D / 4;
+
+// Slot of the item's row `tid`.
+__device__ __forceinline__ int item_fetch_slot(const PrefillParams& p, const ItemDesc& it) {
+  const int64_t t = static_cast<int64_t>(it.st_row) + threadIdx.x;
+  return static_cast<int>(threadIdx.x) < it.st_n && t < p.st_rows ? p.slot_mapping[t] : -1;
+}
+
+// Whether the item's rows are its last keys and in the ring at the end of its loop.
+__device__ __forceinline__ bool rows_in_ring(const ItemDesc& it) {
+  return it.st_row + it.st_n == it.k_start + it.kmax && it.st_n <= it.kmax && it.st_n <= kMaxRingRows;
+}
+
+template <int D>
+__device__ __forceinline__ void put_row_piece(const PrefillParams& p, int kvh, int c, int slot, u32x4 x) {
+  constexpr int PR = kRowPieces<D>;
+  if (slot < 0 || slot >= p.num_slots) return;
+  uint16_t* dst = (c >= PR / 2 ? p.v_cache : p.k_cache) + (static_cast<int64_t>(slot) * p.num_kv_heads + kvh) * D +
+                  8 * (c & (PR / 2 - 1));
+  __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(dst));
+}
+
+template <int D>
+__device__ __forceinline__ void item_store_rows(const PrefillParams& p, const ItemDesc& it, const char* smem_all,
+                                                const int* s_slot) {
+  using Gm = Geom<D>;
+  constexpr int PR = kRowPieces<D>;
+  const int tid = laundered_tid();
+  const int c = tid & (PR - 1);
+  const bool is_v = c >= PR / 2;
+  const int piece = c & (PR / 2 - 1);
+#pragma unroll 4
+  for (int r0 = 0; r0 < it.st_n; r0 += 64 * kWaves / PR) {
+    const int r = r0 + tid / PR;
+    if (r >= it.st_n) break;
+    const int key = it.kmax - it.st_n + r;
+    const int row = key & (kBK - 1);
+    const int at = is_v ? Gm::kVRing + ((piece >> 1) ^ Gm::v_swz(row)) * 32 + (piece & 1) * 16 : (piece ^ Gm::k_swz(row)) * 16;
+    const char* src = smem_all + (key / kBK & (kStages - 1)) * Gm::kTileBytes + row * Gm::RB + at;
+    put_row_piece<D>(p, it.kvh, c, s_slot[r], *reinterpret_cast<const u32x4*>(src));
+  }
+}
+
+// Rows [from, to) of kv heads [h0, h1), for the rows that no item has in its ring: before
+// cu_seqlens_q[0], from cu_seqlens_q[num_seqs] on, past the positions that max_seqlen_q
+// allows, and those of a sequence whose keys are not its own positions.  Normally there
+// are none.
+template <int D>
+__device__ __forceinline__ void store_other_rows(const PrefillParams& p, int64_t from, int64_t to, int h0, int h1) {
+  constexpr int PR = kRowPieces<D>;
+  from = from < 0 ? 0 : from;
+  to = to < p.st_rows ? to : p.st_rows;
+  const int64_t per_row = static_cast<int64_t>(h1 - h0) * PR;
+  for (int64_t i = threadIdx.x; i < (to - from) * per_row; i += 64 * kWaves) {
+    const int64_t t = from + i / per_row;
+    const int rest = static_cast<int>(i % per_row);
+    const int kvh = h0 + rest / PR;
+    const int c = rest & (PR - 1);
+    const bool is_v = c >= PR / 2;
+    const u32x4 x = ld16((is_v ? p.v + t * p.v_row_stride : p.k + t * p.k_row_stride) + kvh * D + 8 * (c & (PR / 2 - 1)));
+    put_row_piece<D>(p, kvh, c, p.slot_mapping[t], x);
+  }
+}
+
+// The rows that the items leave out, stored by the launch's first workgroup.
+template <int D>
+__device__ __forceinline__ void store_rows_outside(const PrefillParams& p, int q_first, int q_last) {
+  if (q_first > 0) store_other_rows<D>(p, 0, q_first, 0, p.num_kv_heads);
+  if (q_last < p.st_rows) store_other_rows<D>(p, q_last, p.st_rows, 0, p.num_kv_heads);
+}
+// The item's rows that it will not store from the ring.
+template <int D>
+__device__ __forceinline__ void store_rows_ahead(const PrefillParams& p, const ItemDesc& it) {
+  const bool ring = rows_in_ring(it);
+  // the last tile that max_seqlen_q allows takes its sequence to the end
+  const bool last = it.tile == p.num_q_tiles - 1 && it.st_n > 0;
+  const int64_t from = static_cast<int64_t>(it.st_row) + (ring ? it.st_n : 0);
+  const int64_t to = last ? static_cast<int64_t>(it.q_start) + it.Lq : static_cast<int64_t>(it.st_row) + it.st_n;
+  if (from < to) store_other_rows<D>(p, from, to, it.kvh, it.kvh + 1);
+}
+
 // Run work item `it` on the whole workgroup.  Its Q operands (qop) and the
 // copies of its tiles 0 and 1 were issued before (item_fetch_q,
 // item_fetch_tiles).  When `next` is valid, this issues next's Q loads into
@@ -574,11 +675,13 @@ __device__ __forceinline__ void item_fetch_tiles(const PrefillParams& p, char* s
 // after the epilogue's barrier, so their latency overlaps the epilogue; the
 // epilogue's transpose therefore uses ring stages 2 and 3 only.  SPLIT: the
 // item may be one key half, merged at the end (merge_key_halves); only the
-// direct grid splits, so the persistent grid's code carries no merge.
-template <bool PAGED, int D, bool SPLIT>
+// direct grid splits, so the persistent grid's code carries no merge.  STORE: the
+// item's rows go from the ring to the caches after the loop; `slot` is this thread's
+// row's slot, fetched before like the Q operands.
+template <bool PAGED, int D, bool SPLIT, bool STORE>
 __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_all, const ItemDesc& item,
                                             bf16x8 (&qop)[D / 16], const ItemDesc& next, uint32_t* claim_ctr,
-                                            uint32_t& claim) {
+                                            uint32_t& claim, int* s_slot, int& slot) {
   using Gm = Geom<D>;
   constexpr int RB = Gm::RB;
   constexpr int KP = Gm::KP;
@@ -821,6 +924,9 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   // the compiler would then keep those loads pending into the loop and wait
   // for all vector memory there -- which, unknown to it, also drains the tile
   // copies in flight -- on every step.
+  if constexpr (STORE) {
+    if (tid < item.st_n) s_slot[tid] = slot;  // read after the loop's barriers
+  }
   barrier_lds();
   if (2 < ntiles) {
     stg.template copy_part<0, P>(item, stage(2), c_ptr, 2);
@@ -840,7 +946,13 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   // ---- epilogue: normalise, transpose through LDS, write whole rows --------
   // The next item's Q operands first: the last QK has been issued, so qop is
   // free, and the loads have the epilogue to land.
-  if (next.valid) item_fetch_q<D>(p, next, qop);
+  if (next.valid) {
+    item_fetch_q<D>(p, next, qop);
+    if constexpr (STORE) slot = item_fetch_slot(p, next);
+  }
+  if constexpr (STORE) {
+    if (rows_in_ring(item)) item_store_rows<D>(p, item, smem_all, s_slot);
+  }
   float l = sum_across_halves(l_run[0] + l_run[1]);
   if constexpr (SPLIT) {
     if (item.split_slot >= 0 && !merge_key_halves<D>(p, smem_all, item.split_slot, acc, m_run, l)) return;
@@ -887,9 +999,12 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // on the same XCD (and its L2) whenever gridDim.x is a multiple of 8.  Tiles
 // past a sequence's end exit at once.  Used when the persistent grid's tables
 // would not fit its LDS.
-template <bool PAGED, int D>
+template <bool PAGED, int D, bool STORE>
 __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
+  if constexpr (STORE) {
+    if (blockIdx.x == 0 && blockIdx.y == 0) store_rows_outside<D>(p, p.cu_q[0], p.cu_q[p.num_seqs]);
+  }
   int s, kvh, tile, half = 0, pair = -1;
   if (p.split_tiles > 0) {
     // key halving: the compact grid (the real items first, heaviest first;
@@ -910,13 +1025,17 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillPara
   ItemDesc it = item_desc(p, p.cu_q, p.cu_k, s, kvh, tile);
   if (!it.valid) return;
   if (pair >= 0) key_half<PAGED>(p, it, half, pair * p.num_kv_heads + kvh);
+  __shared__ int s_slot[STORE ? kRows : 1];
+  int slot = -1;
+  if constexpr (STORE) store_rows_ahead<D>(p, it);
   bf16x8 qop[D / 16];
   item_fetch_q<D>(p, it, qop);
   item_fetch_tiles<PAGED, D>(p, smem_all, it);
+  if constexpr (STORE) slot = item_fetch_slot(p, it);
   ItemDesc none{};
   none.valid = false;
   uint32_t unused = 0;
-  prefill_run<PAGED, D, true>(p, smem_all, it, qop, none, nullptr, unused);
+  prefill_run<PAGED, D, true, STORE>(p, smem_all, it, qop, none, nullptr, unused, s_slot, slot);
 }
 
 // Persistent grid: one workgroup per CU walks the real work items.
@@ -968,13 +1087,14 @@ __device__ __forceinline__ int find_seq(const int* s_ntq, int S, int t, int rank
   return -1;
 }
 
-template <bool PAGED, int D, bool QUEUE>
+template <bool PAGED, int D, bool QUEUE, bool STORE>
 __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
   __shared__ int s_ntq[kPersistMaxSeqs];           // query tiles of each sequence
   __shared__ int s_start[kPersistMaxTiles + 1];    // first item of each tile level (level T_max: total)
   __shared__ int s_cu[2][kPersistMaxSeqs + 1];     // cu_seqlens_q and cu_seqlens_k
   __shared__ uint32_t s_claim;                     // the queue claim, broadcast by thread 0
+  __shared__ int s_slot[STORE ? kRows : 1];        // cache slots of the item's rows
   const int tid = threadIdx.x;
   const int S = p.num_seqs;
   const int T = p.num_q_tiles;
@@ -1046,6 +1166,9 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
   }
   __syncthreads();
   const int total = s_start[T];
+  if constexpr (STORE) {
+    if (g == 0) store_rows_outside<D>(p, s_cu[0][0], s_cu[0][S]);
+  }
   // Table item `item` (every item below `total` is a real tile: its sequence
   // has more than t query tiles), or an invalid descriptor past the end.
   auto desc_of = [&](int item) {
@@ -1075,8 +1198,10 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
     return;
   }
   bf16x8 qop[D / 16];
+  int slot = -1;
   item_fetch_q<D>(p, cur, qop);
   item_fetch_tiles<PAGED, D>(p, smem_all, cur);
+  if constexpr (STORE) slot = item_fetch_slot(p, cur);
   for (int round = 1;; ++round) {
     // the next item is located (from the LDS tables) while this one's
     // first copies are in flight; its own first copies start in this one's
@@ -1091,7 +1216,8 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
       const int64_t item64 = static_cast<int64_t>(round) * NW + q;
       nxt = desc_of(item64 < total ? static_cast<int>(item64) : total);
     }
-    prefill_run<PAGED, D, false>(p, smem_all, cur, qop, nxt, claim_ctr, claim);
+    if constexpr (STORE) store_rows_ahead<D>(p, cur);
+    prefill_run<PAGED, D, false, STORE>(p, smem_all, cur, qop, nxt, claim_ctr, claim, s_slot, slot);
     if (!nxt.valid) break;
     cur = nxt;
   }
@@ -1124,30 +1250,54 @@ constexpr int kSplitDen = 5;
 constexpr int kSplitMin = 8;
 constexpr int kSplitMaxPageTiles = 8;  // paged key halving for block sizes up to 512
 
-hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seqlen_k, hipStream_t stream) {
-  if (p0.num_seqs <= 0 || max_seqlen_q <= 0) return hipSuccess;
+hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seqlen_k, hipStream_t stream,
+                          const StoreParams* store, int store_vec) {
+  const bool nothing = p0.num_seqs <= 0 || max_seqlen_q <= 0;
   PrefillParams p = p0;
   p.positions_per_tile = prefill_positions_per_tile(p.group);
-  p.num_q_tiles = (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile;
+  p.num_q_tiles = nothing ? 0 : (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile;
   // Persistent grid when there are enough items to balance; with at most two
   // per CU its table set-up (one more dependent global load and a few
   // barriers) costs more than it saves (measured on config 2).
   const int64_t max_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
   const int cus = device_cu_count();
-  if (p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles && max_items > 2 * int64_t{cus}) {
-    // one workgroup per CU (the ring takes most of a CU's LDS); the work queue
-    // needs whole XCD lanes
-    const unsigned nw = static_cast<unsigned>(cus);
+  const bool persistent =
+      p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles && max_items > 2 * int64_t{cus};
+  // one workgroup per CU (the ring takes most of a CU's LDS); the work queue
+  // needs whole XCD lanes
+  const unsigned nw = static_cast<unsigned>(cus);
+  const bool queue = p.queue != nullptr && nw % kPrefillQueueLanes == 0;
+  // The store rides on the launch when the keys are the fresh rows (the attention then
+  // reads no cache), an item's rows fit the ring's last tiles (a GQA group of one has
+  // 256), and the static item order is not in use.
+  const bool fuse = store != nullptr && !nothing && !p.block_table && store->cache_dtype == 0 && store_vec == 16 &&
+                    p.positions_per_tile <= kMaxRingRows && (!persistent || queue);
+  if (fuse) {
+    p.k_cache = static_cast<uint16_t*>(store->k_cache);
+    p.v_cache = static_cast<uint16_t*>(store->v_cache);
+    p.slot_mapping = store->slot_mapping;
+    p.num_slots = store->num_slots;
+    p.st_rows = store->num_tokens;
+  } else if (store != nullptr) {
+    const hipError_t e = launch_store_kvcache(*store, store_vec, stream);
+    if (e != hipSuccess) return e;
+  }
+  if (nothing) return hipSuccess;
+  if (persistent) {
     const dim3 grid(nw);
-    const bool queue = p.queue != nullptr && nw % kPrefillQueueLanes == 0;
-#define NVA_PERSIST(PG, DD)                                                                                  \
-  do {                                                                                                       \
-    if (queue)                                                                                               \
-      hipLaunchKernelGGL((varlen_prefill_persistent_kernel<PG, DD, true>), grid, dim3(kThreads), 0, stream, p); \
-    else                                                                                                     \
-      hipLaunchKernelGGL((varlen_prefill_persistent_kernel<PG, DD, false>), grid, dim3(kThreads), 0, stream, p); \
+#define NVA_PERSIST(PG, DD)                                                                                         \
+  do {                                                                                                              \
+    if (queue)                                                                                                      \
+      hipLaunchKernelGGL((varlen_prefill_persistent_kernel<PG, DD, true, false>), grid, dim3(kThreads), 0, stream, p); \
+    else                                                                                                            \
+      hipLaunchKernelGGL((varlen_prefill_persistent_kernel<PG, DD, false, false>), grid, dim3(kThreads), 0, stream, p); \
   } while (0)
-    if (p.head_dim == 64) {
+    if (fuse) {
+      if (p.head_dim == 64)
+        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<false, 64, true, true>), grid, dim3(kThreads), 0, stream, p);
+      else
+        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<false, 128, true, true>), grid, dim3(kThreads), 0, stream, p);
+    } else if (p.head_dim == 64) {
       if (p.block_table) NVA_PERSIST(true, 64);
       else NVA_PERSIST(false, 64);
     } else {
@@ -1176,17 +1326,18 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   const dim3 grid = p.split_tiles > 0
                         ? dim3(static_cast<unsigned>(max_items + pairs_split * p.num_kv_heads))
                         : dim3(static_cast<unsigned>(p.num_seqs * p.num_kv_heads), static_cast<unsigned>(p.num_q_tiles));
+#define NVA_DIRECT(PG, DD, ST) \
+  hipLaunchKernelGGL((varlen_prefill_kernel<PG, DD, ST>), grid, dim3(kThreads), 0, stream, p)
   if (p.head_dim == 64) {
-    if (p.block_table)
-      hipLaunchKernelGGL((varlen_prefill_kernel<true, 64>), grid, dim3(kThreads), 0, stream, p);
-    else
-      hipLaunchKernelGGL((varlen_prefill_kernel<false, 64>), grid, dim3(kThreads), 0, stream, p);
+    if (p.block_table) NVA_DIRECT(true, 64, false);
+    else if (fuse) NVA_DIRECT(false, 64, true);
+    else NVA_DIRECT(false, 64, false);
   } else {
-    if (p.block_table)
-      hipLaunchKernelGGL((varlen_prefill_kernel<true, 128>), grid, dim3(kThreads), 0, stream, p);
-    else
-      hipLaunchKernelGGL((varlen_prefill_kernel<false, 128>), grid, dim3(kThreads), 0, stream, p);
+    if (p.block_table) NVA_DIRECT(true, 128, false);
+    else if (fuse) NVA_DIRECT(false, 128, true);
+    else NVA_DIRECT(false, 128, false);
   }
+#undef NVA_DIRECT
   return hipGetLastError();
 }
 

@@ -186,6 +186,17 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
     kv head) are first gathered into packed bf16 rows, dequantised
     (nva_gather_kv), and the packed prefill runs on those.  That needs
     cu_seqlens_k[s+1] - cu_seqlens_k[s] <= max_seqlen_k, as flash-attn does."""
+    qa, kv, pages, rest, (out, *_rows) = _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k,
+                                                       softmax_scale, causal, block_table, k_scale, v_scale)
+    _capi.check(_capi.load().nva_prefill(*qa, *kv, *pages, *rest))
+    return out
+
+
+def _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale, causal,
+                  block_table, k_scale, v_scale):
+    """Checks of the prefill call and its nva_prefill arguments in four groups (q, k and v,
+    block table, the rest), with the tensors they point into that the call made; an fp8
+    cache is gathered here."""
     if not causal:
         raise RuntimeError("only causal=True is implemented (the only mode attention.py uses)")
     total_q, nh, d = q.shape
@@ -244,15 +255,33 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
         k_row, v_row = k.stride(0), v.stride(0)
         bt_ptr, bt_stride, max_blocks, block_size, num_blocks = None, 0, 0, 0, 0
     _check_device(q.device, k=k, v=v, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k, block_table=block_table)
-    lib = _capi.load()
     stream = _stream(q)
     ws = _prefill_workspace(q.device, stream)
-    _capi.check(lib.nva_prefill(
-        q.data_ptr(), q.stride(0), k.data_ptr(), k_row, v.data_ptr(), v_row,
-        bt_ptr, bt_stride, max_blocks, block_size, num_blocks,
-        cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), num_seqs, int(max_seqlen_q), int(max_seqlen_k),
-        nh, nkv, d, float(softmax_scale), out.data_ptr(), out.stride(0),
-        _ptr(ws), 0 if ws is None else ws.numel(), stream))
+    return (q.data_ptr(), q.stride(0)), (k.data_ptr(), k_row, v.data_ptr(), v_row), \
+        (bt_ptr, bt_stride, max_blocks, block_size, num_blocks), \
+        (cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), num_seqs, int(max_seqlen_q), int(max_seqlen_k),
+         nh, nkv, d, float(softmax_scale), out.data_ptr(), out.stride(0),
+         _ptr(ws), 0 if ws is None else ws.numel(), stream), (out, k, v)
+
+
+def _store_and_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                       slot_mapping: torch.Tensor, max_seqlen_q: int, cu_seqlens_q: torch.Tensor, max_seqlen_k: int,
+                       cu_seqlens_k: torch.Tensor, softmax_scale: float, k_scale: torch.Tensor | None,
+                       v_scale: torch.Tensor | None) -> torch.Tensor:
+    """The prefill branch of Attention.forward without a cached prefix as one call:
+    store_kvcache of the fresh rows (attention.py:32-39), then flash_attn_varlen_func over
+    those rows (attention.py:67-73), which never reads the caches (nva_store_prefill).
+    A call that the attention refuses still stores, as the two calls would."""
+    N, nkv, d, code = _check_store(k, v, k_cache, v_cache, slot_mapping, k_scale, v_scale)
+    try:
+        qa, kv, _, rest, (out, *_rows) = _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k,
+                                                       softmax_scale, True, None, None, None)
+        _capi.check(_capi.load().nva_store_prefill(
+            k_cache.data_ptr(), v_cache.data_ptr(), k_cache.numel() // (nkv * d), slot_mapping.data_ptr(), N, code,
+            _ptr(k_scale), _ptr(v_scale), *qa, q.shape[0], *kv, *rest))
+    except Exception:
+        store_kvcache(k, v, k_cache, v_cache, slot_mapping, k_scale, v_scale)
+        raise
     return out
 
 
@@ -371,6 +400,11 @@ class Attention(nn.Module):
             o = store_and_decode(q.unsqueeze(1), k, v, k_cache, v_cache, context.slot_mapping,
                                  context.context_lens, context.block_tables, softmax_scale=self.scale,
                                  k_scale=self.k_scale, v_scale=self.v_scale)
+            return o.view(-1, self.num_heads * self.head_dim)
+        if context.is_prefill and bound and context.block_tables is None:  # no cached prefix: k and v are the keys
+            o = _store_and_prefill(q, k, v, k_cache, v_cache, context.slot_mapping, context.max_seqlen_q,
+                                   context.cu_seqlens_q, context.max_seqlen_k, context.cu_seqlens_k, self.scale,
+                                   self.k_scale, self.v_scale)
             return o.view(-1, self.num_heads * self.head_dim)
         if bound:
             store_kvcache(k, v, k_cache, v_cache, context.slot_mapping, self.k_scale, self.v_scale)
