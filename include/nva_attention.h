@@ -119,6 +119,25 @@ int nva_prefill(const void* q, int64_t q_row_stride,
                 void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * nva_prefill over the pages of an fp8 e4m3fn cache (one float32 scale per kv head; the
+ * reference's caches hold the model dtype only): the pages are converted to bf16 as they are
+ * staged, k_scale multiplies the scores and v_scale the output.  Arguments and results as
+ * nva_prefill with block_table; head_dim 128.  nva_gather_kv and a packed nva_prefill serve
+ * the rest (other head dims and block sizes; many query tiles per key).
+ */
+int nva_prefill_fp8(const void* q, int64_t q_row_stride,
+                    const void* k_cache, const void* v_cache,
+                    const float* k_scale, const float* v_scale,
+                    const int32_t* block_table, int64_t bt_row_stride,
+                    int32_t max_blocks_per_seq, int32_t block_size, int64_t num_blocks,
+                    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                    int32_t num_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k,
+                    int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                    float softmax_scale,
+                    void* out, int64_t out_row_stride,
+                    void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * One prefill step of Attention.forward without a cached prefix (attention.py:58-73): the store
  * of the fresh rows (nva_store_kvcache with key = k, value = v) followed by the packed prefill
  * over them (nva_prefill with block_table NULL), with the results of the two calls.  The

@@ -137,14 +137,15 @@ int nva_store_kvcache(const void* key, int64_t key_row_stride, const void* value
 namespace {
 
 // nva_prefill's body.  `store`: the store that comes before it (null: none), fused into the
-// launch by launch_prefill where it can be.
+// launch by launch_prefill where it can be.  k_scale/v_scale: the paged caches are fp8.
 int prefill_impl(const void* q, int64_t q_row_stride, const void* k, int64_t k_row_stride, const void* v,
                 int64_t v_row_stride, const int32_t* block_table, int64_t bt_row_stride,
                 int32_t max_blocks_per_seq, int32_t block_size, int64_t num_blocks,
                 const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int32_t num_seqs,
                 int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads, int32_t num_kv_heads,
                 int32_t head_dim, float softmax_scale, void* out, int64_t out_row_stride, void* workspace,
-                int64_t workspace_bytes, void* stream, const nva::StoreParams* store = nullptr, int store_vec = 0) {
+                int64_t workspace_bytes, void* stream, const nva::StoreParams* store = nullptr, int store_vec = 0,
+                const float* k_scale = nullptr, const float* v_scale = nullptr) {
   if (head_dim != 128 && head_dim != 64)
     return fail(NVA_ERR_UNSUPPORTED, "head_dim %d not supported (64 or 128)", head_dim);
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
@@ -193,6 +194,8 @@ int prefill_impl(const void* q, int64_t q_row_stride, const void* k, int64_t k_r
   p.q = static_cast<const uint16_t*>(q);
   p.k = static_cast<const uint16_t*>(k);
   p.v = static_cast<const uint16_t*>(v);
+  p.k_scale = k_scale;
+  p.v_scale = v_scale;
   p.block_table = block_table;
   p.cu_q = cu_seqlens_q;
   p.cu_k = cu_seqlens_k;
@@ -277,6 +280,26 @@ int nva_store_prefill(void* k_cache, void* v_cache, int64_t num_slots, const int
   return prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, nullptr, 0, 0, 0, 0, cu_seqlens_q,
                       cu_seqlens_k, num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim,
                       softmax_scale, out, out_row_stride, workspace, workspace_bytes, stream, apart ? nullptr : &sp, vec);
+}
+
+int nva_prefill_fp8(const void* q, int64_t q_row_stride, const void* k_cache, const void* v_cache, const float* k_scale,
+                    const float* v_scale, const int32_t* block_table, int64_t bt_row_stride, int32_t max_blocks_per_seq,
+                    int32_t block_size, int64_t num_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                    int32_t num_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t num_heads,
+                    int32_t num_kv_heads, int32_t head_dim, float softmax_scale, void* out, int64_t out_row_stride,
+                    void* workspace, int64_t workspace_bytes, void* stream) {
+  if (head_dim != 128) return fail(NVA_ERR_UNSUPPORTED, "fp8 paged prefill supports head_dim 128 only (got %d)", head_dim);
+  if (num_seqs > 0 && max_seqlen_q > 0) {
+    if (!block_table || !k_scale || !v_scale)
+      return fail(NVA_ERR_INVALID_ARGUMENT, "fp8 paged prefill needs block_table, k_scale and v_scale");
+    if (!aligned(k_scale, 4) || !aligned(v_scale, 4))
+      return fail(NVA_ERR_INVALID_ARGUMENT, "scales must be 4-byte aligned");
+  }
+  const int64_t row = static_cast<int64_t>(num_kv_heads) * head_dim;
+  return prefill_impl(q, q_row_stride, k_cache, row, v_cache, row, block_table, bt_row_stride, max_blocks_per_seq,
+                      block_size, num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q, max_seqlen_k,
+                      num_heads, num_kv_heads, head_dim, softmax_scale, out, out_row_stride, workspace, workspace_bytes,
+                      stream, nullptr, 0, k_scale, v_scale);
 }
 
 int64_t nva_prefill_workspace_bytes(void) { return nva::kPrefillWorkspaceBytes; }

@@ -1,7 +1,8 @@
 // Paged cache -> packed rows: the keys and values of every sequence, gathered
 // through its block table and written as bf16 rows at cu_seqlens_k[s] + j.
-// This is how a prefix-cached prefill (nanovllm/layers/attention.py:68-73)
-// reads an fp8 e4m3fn cache: the rows are dequantised here (x = e4m3 * scale
+// This is how a prefix-cached prefill (nanovllm/layers/attention.py:68-73) with
+// many query tiles per key reads an fp8 e4m3fn cache (one with few converts the
+// pages as it stages them): the rows are dequantised here (x = e4m3 * scale
 // of the kv head, rounded to bf16) and the packed prefill kernel runs on them,
 // so the MFMA prefill keeps its global->LDS copies.  A bf16 cache is copied
 // bit for bit.

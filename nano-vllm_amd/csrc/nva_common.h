@@ -137,6 +137,21 @@ __device__ __forceinline__ uint32_t fp8x2_to_bf16x2(uint32_t w) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// 16 fp8 -> two 8 x bf16 vectors.
+__device__ __forceinline__ void fp8x16_to_bf16(u32x4 w, bf16x8& lo, bf16x8& hi) {
+  u32x4 a, b;
+  a[0] = fp8x2_to_bf16x2<false>(w[0]);
+  a[1] = fp8x2_to_bf16x2<true>(w[0]);
+  a[2] = fp8x2_to_bf16x2<false>(w[1]);
+  a[3] = fp8x2_to_bf16x2<true>(w[1]);
+  b[0] = fp8x2_to_bf16x2<false>(w[2]);
+  b[1] = fp8x2_to_bf16x2<true>(w[2]);
+  b[2] = fp8x2_to_bf16x2<false>(w[3]);
+  b[3] = fp8x2_to_bf16x2<true>(w[3]);
+  lo = as_bf16x8(a);
+  hi = as_bf16x8(b);
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Cross-lane xor shuffle within the 64-lane wavefront.

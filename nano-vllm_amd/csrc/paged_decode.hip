@@ -73,21 +73,6 @@ __device__ __forceinline__ void transpose_v_fp8(const u32x2 (&vr)[8], bf16x8 (&v
   for (int j = 0; j < 8; ++j) vt[j] = as_bf16x8(o[j]);
 }
 
-// 16 fp8 -> two 8 x bf16 MFMA operands.
-__device__ __forceinline__ void fp8x16_to_ops(u32x4 w, bf16x8& lo, bf16x8& hi) {
-  u32x4 a, b;
-  a[0] = fp8x2_to_bf16x2<false>(w[0]);
-  a[1] = fp8x2_to_bf16x2<true>(w[0]);
-  a[2] = fp8x2_to_bf16x2<false>(w[1]);
-  a[3] = fp8x2_to_bf16x2<true>(w[1]);
-  b[0] = fp8x2_to_bf16x2<false>(w[2]);
-  b[1] = fp8x2_to_bf16x2<true>(w[2]);
-  b[2] = fp8x2_to_bf16x2<false>(w[3]);
-  b[3] = fp8x2_to_bf16x2<true>(w[3]);
-  lo = as_bf16x8(a);
-  hi = as_bf16x8(b);
-}
-
 }  // namespace
 
 // Raw loads of one 32-key step for one kv head (see the file comment for the
@@ -254,7 +239,7 @@ __device__ __forceinline__ void compute_step(StepRegs<FP8>& r, int nvalid, int g
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int u = 0; u < D / 64; ++u) fp8x16_to_ops(r.k[t][u], kop[t][2 * u], kop[t][2 * u + 1]);
+      for (int u = 0; u < D / 64; ++u) fp8x16_to_bf16(r.k[t][u], kop[t][2 * u], kop[t][2 * u + 1]);
   }
   f32x4 st[2];
 #pragma unroll

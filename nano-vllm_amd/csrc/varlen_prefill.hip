@@ -38,6 +38,7 @@
 // (so p <= 2^kTau), which makes the rescale of the accumulators rare.  Masks
 // are evaluated only on tiles that cross the causal diagonal or the key end.
 #include <algorithm>
+#include <type_traits>
 
 #include "nva_common.h"
 #include "nva_kernels.h"
@@ -120,6 +121,50 @@ __device__ __forceinline__ StageLane<Geom<D>::P> stage_lane(int w, int lane, int
   return d;
 }
 
+// Staging of an fp8 e4m3fn tile (kKvFp8): the rows go through registers, converted to
+// bf16 on the way (exactly: the scales are applied to Q and to the output), so the LDS
+// tiles and the whole loop are those of a bf16 cache, at half the bytes from memory.
+// Against a gather into bf16 rows before a packed launch: 6 sequences of 100-1500 tokens
+// after 1536 cached ones, heads 32/8, store included, 166.0 -> 149.5 us; the conversion
+// (16 instructions and 4 LDS writes a lane and tile) costs the loop ~3%.
+// Wave w moves 16 rows of K (w < 4) or V; per load, lane l carries 16 elements (two of a
+// row's 16-byte LDS pieces) of row l / 8.  Row `row[u]` of load u, at byte `off[u]` from the
+// tile's first key; its first piece lands at `lds[u]` of the tile's stage, the second at
+// lds[u] ^ 16.
+struct StageLane8 {
+  int row[2];
+  uint32_t off[2];
+  uint32_t lds[2];
+};
+
+template <int D>
+__device__ __forceinline__ StageLane8 stage_lane8(int w, int lane, int64_t stride) {
+  using Gm = Geom<D>;
+  static_assert(D == 128, "eight lanes of 16 elements per row");
+  StageLane8 d;
+  const int c = lane & 7;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int row = 16 * (w & 3) + 8 * u + (lane >> 3);
+    d.row[u] = row;
+    d.off[u] = static_cast<uint32_t>(row * stride + 16 * c);
+    d.lds[u] = static_cast<uint32_t>(row * Gm::RB + (w < 4 ? ((2 * c) ^ Gm::k_swz(row)) * 16
+                                                           : Gm::kVRing + (c ^ Gm::v_swz(row)) * 32));
+  }
+  return d;
+}
+
+// A tile's fp8 bytes of one lane on their way to LDS.
+struct Raw8 {
+  u32x4 x[2];
+};
+
+// How an item's keys and values are held: fresh bf16 rows, pages of a bf16 cache, pages of
+// an fp8 e4m3fn cache.
+constexpr int kKvPacked = 0;
+constexpr int kKvPaged = 1;
+constexpr int kKvFp8 = 2;
+
 typedef const __attribute__((address_space(4))) int32_t const_i32;
 
 // Block id of the page holding key kb (-1 past the mb entries of the table row
@@ -136,8 +181,8 @@ __device__ __forceinline__ int page_of(const PrefillParams& p, const_i32* bt, in
 // those keys are not masked (the result of such a sequence is unspecified,
 // other sequences are unaffected).  Masking them costs the loop ~3% (scalar
 // state per ring stage), so only decode masks them.
-template <bool PAGED>
-__device__ __forceinline__ const char* tile_base(const PrefillParams& p, const uint16_t* base, int64_t stride, int page,
+template <bool PAGED, class Elem>
+__device__ __forceinline__ const char* tile_base(const PrefillParams& p, const Elem* base, int64_t stride, int page,
                                                  int k_start, int kb) {
   int64_t slot0;
   if constexpr (PAGED) {
@@ -527,13 +572,16 @@ __device__ __forceinline__ void item_fetch_q(const PrefillParams& p, const ItemD
 
 // Per-wave staging constants of item `it`'s K/V tiles (waves 0..3 copy K,
 // 4..7 copy V).
-template <bool PAGED, int D>
+template <int KV, int D>
 struct ItemStaging {
+  static constexpr bool PAGED = KV != kKvPacked;
+  static constexpr bool FP8 = KV == kKvFp8;
   const_i32* bt;
   int mb;  // entries of the block-table row from bt on
-  const uint16_t* dbase;
+  typedef typename std::conditional<FP8, uint8_t, uint16_t>::type Elem;
+  const Elem* dbase;
   int64_t dstride;
-  StageLane<Geom<D>::P> dl;
+  typename std::conditional<FP8, StageLane8, StageLane<Geom<D>::P>>::type dl;
   int v_skip;
   int w;
 
@@ -544,9 +592,12 @@ struct ItemStaging {
     const bool k_wave = w < 4;
     bt = PAGED ? (const_i32*)(p.block_table + static_cast<int64_t>(it.s) * p.bt_row_stride + it.bt_off) : nullptr;
     mb = p.max_blocks - it.bt_off;
-    dbase = (k_wave ? p.k : p.v) + it.kvh * D;
+    dbase = reinterpret_cast<const Elem*>(k_wave ? p.k : p.v) + it.kvh * D;
     dstride = k_wave ? p.k_row_stride : p.v_row_stride;
-    dl = stage_lane<D>(w, tid & 63, dstride);
+    if constexpr (FP8)
+      dl = stage_lane8<D>(w, tid & 63, dstride);
+    else
+      dl = stage_lane<D>(w, tid & 63, dstride);
     v_skip = k_wave ? 0 : Gm::kVRing - Gm::kTileBytes;
   }
   // first key of tile t in global memory
@@ -561,15 +612,43 @@ struct ItemStaging {
   __device__ __forceinline__ void copy_part(const ItemDesc& it, char* st, const char* src, int t) const {
     dma_tile<Geom<D>::P, U0, U1>(st, src, dl, t * kBK, it.kmax, w, v_skip);
   }
+  // fp8: load this lane's part of tile t (keys at or past kmax: the tile's first key, as
+  // dma_tile), and write it to the tile's stage
+  __device__ __forceinline__ void load8(const ItemDesc& it, const char* src, int t, Raw8& r) const {
+    const int nrow = it.kmax - t * kBK;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t col = 16u * (static_cast<uint32_t>(laundered_tid()) & 7u);
+      r.x[u] = ld16(src + (dl.row[u] < nrow ? dl.off[u] : col));
+    }
+  }
+  __device__ __forceinline__ void write8(char* st, const Raw8& r) const {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      bf16x8 lo, hi;
+      fp8x16_to_bf16(r.x[u], lo, hi);
+      *reinterpret_cast<u32x4*>(st + dl.lds[u]) = as_u32x4(lo);
+      *reinterpret_cast<u32x4*>(st + (dl.lds[u] ^ 16u)) = as_u32x4(hi);
+    }
+  }
 };
 
-// Start the copies of item `it`'s tiles 0 and 1 into ring stages 0 and 1.
-template <bool PAGED, int D>
-__device__ __forceinline__ void item_fetch_tiles(const PrefillParams& p, char* smem_all, const ItemDesc& it) {
-  const ItemStaging<PAGED, D> st(p, it);
+// Start the copies of item `it`'s tiles 0 and 1 into ring stages 0 and 1 (fp8: the loads
+// into raw; the prologue writes them).
+template <int KV, int D>
+__device__ __forceinline__ void item_fetch_tiles(const PrefillParams& p, char* smem_all, const ItemDesc& it,
+                                                 Raw8 (&raw)[2]) {
+  const ItemStaging<KV, D> st(p, it);
+  constexpr bool PAGED = KV != kKvPacked;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
-    if (t < it.ntiles) st.copy(p, it, smem_all + t * Geom<D>::kTileBytes, PAGED ? page_of(p, st.bt, st.mb, t * kBK) : 0, t);
+    if (t < it.ntiles) {
+      const int page = PAGED ? page_of(p, st.bt, st.mb, t * kBK) : 0;
+      if constexpr (KV == kKvFp8)
+        st.load8(it, st.tile(p, it, page, t), t, raw[t]);
+      else
+        st.copy(p, it, smem_all + t * Geom<D>::kTileBytes, page, t);
+    }
 }
 
 // The store fused into a packed prefill: every item also writes the cache rows of its
@@ -678,11 +757,15 @@ __device__ __forceinline__ void store_rows_ahead(const PrefillParams& p, const I
 // direct grid splits, so the persistent grid's code carries no merge.  STORE: the
 // item's rows go from the ring to the caches after the loop; `slot` is this thread's
 // row's slot, fetched before like the Q operands.
-template <bool PAGED, int D, bool SPLIT, bool STORE>
+// KV == kKvFp8: raw[0] and raw[1] are
+// the bytes of tiles 0 and 1, loaded before like the Q operands.
+template <int KV, int D, bool SPLIT, bool STORE>
 __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_all, const ItemDesc& item,
                                             bf16x8 (&qop)[D / 16], const ItemDesc& next, uint32_t* claim_ctr,
-                                            uint32_t& claim, int* s_slot, int& slot) {
+                                            uint32_t& claim, int* s_slot, int& slot, Raw8 (&raw)[2]) {
   using Gm = Geom<D>;
+  constexpr bool PAGED = KV != kKvPacked;
+  constexpr bool FP8 = KV == kKvFp8;
   constexpr int RB = Gm::RB;
   constexpr int KP = Gm::KP;
   constexpr int P = Gm::P;
@@ -730,7 +813,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   float m_run = 0.f;  // row maximum (log2 units); scores leave the QK product relative to it
   f32x16 negm = f32x16{};  // -m_run in every register: the C operand of the QK chain
   float l_run[2] = {0.f, 0.f};  // this lane's half of the row sum, two dot2 chains
-  const float sl2 = p.scale_log2;
+  const float sl2 = FP8 ? p.scale_log2 * p.k_scale[item.kvh] : p.scale_log2;
 
   // Per-lane LDS byte offsets of the MFMA operand reads inside a stage; the
   // 32-key half (sub), PV MFMA (u) and 4-key block (eb) add constants.
@@ -747,7 +830,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
     vaddr[jd] = Gm::kVRing + (4 * h + (jl >> 2)) * RB +
                 ((2 * jd + ((lane >> 4) & 1)) ^ Gm::v_swz(jl >> 2)) * 32 + 8 * (jl & 3);
 
-  const ItemStaging<PAGED, D> stg(p, item);
+  const ItemStaging<KV, D> stg(p, item);
   (void)s;
   (void)k_start;
   (void)kvh;
@@ -859,7 +942,8 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   // outside the pool redirects to slot 0).  Block sizes are multiples of 64,
   // so a tile never straddles two pages, and the loop needs no division and
   // no 64-bit multiply per tile.
-  const int64_t tile_step = static_cast<int64_t>(kBK) * stg.dstride * 2;
+  constexpr int EB = FP8 ? 1 : 2;  // bytes per cache element
+  const int64_t tile_step = static_cast<int64_t>(kBK) * stg.dstride * EB;
   const int tpp = PAGED ? p.block_size / kBK : 1;  // tiles per page
   const uint32_t nb32 = p.num_blocks > 0x7fffffff ? 0x7fffffffu : static_cast<uint32_t>(p.num_blocks);
   auto page_at = [&](int idx) { return idx < stg.mb ? stg.bt[idx] : -1; };
@@ -886,9 +970,24 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
       c_ptr += tile_step;
     }
   };
-  auto tile_iter = [&](int it, const char* cur, const char* nxt, char* fill) {
+  // fp8: tile it+2's bytes, loaded one tile ago, are converted into the stage that tile
+  // it-2 left (visible after the next tile's barrier, where its first QK needs them), and
+  // tile it+3's are loaded in their place.
+  auto tile_iter = [&](int it, const char* cur, const char* nxt, char* fill, char* fill2) {
     const int kb = it * kBK;
     step(s0, s1, kb, cur, cur + 32 * RB);
+    if constexpr (FP8) {
+      (void)fill;
+      barrier_lds();
+      if (it + 2 < ntiles) stg.write8(fill2, raw[0]);
+      if (it + 3 < ntiles) {
+        stg.load8(item, c_ptr, it + 3, raw[0]);
+        advance();
+      }
+      step(s1, s0, kb + 32, cur + 32 * RB, nxt);
+      return;
+    }
+    (void)fill2;
     if (it + 2 < ntiles)
       wait_vmem<P>();  // tile it+2's copy may stay in flight
     else
@@ -897,12 +996,16 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
     // tile it+3's copy in two halves, one on each side of the second step, so
     // its LDS writes do not all land at once among the operand reads
     const char* src3 = c_ptr;
-    if (it + 3 < ntiles) {
-      stg.template copy_part<0, P / 2>(item, fill, src3, it + 3);
-      advance();
+    if constexpr (!FP8) {
+      if (it + 3 < ntiles) {
+        stg.template copy_part<0, P / 2>(item, fill, src3, it + 3);
+        advance();
+      }
     }
     step(s1, s0, kb + 32, cur + 32 * RB, nxt);
-    if (it + 3 < ntiles) stg.template copy_part<P / 2, P>(item, fill, src3, it + 3);
+    if constexpr (!FP8) {
+      if (it + 3 < ntiles) stg.template copy_part<P / 2, P>(item, fill, src3, it + 3);
+    }
   };
 
   // prologue: tiles 0 and 1 (copies issued before this call) and the Q
@@ -927,9 +1030,18 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   if constexpr (STORE) {
     if (tid < item.st_n) s_slot[tid] = slot;  // read after the loop's barriers
   }
+  if constexpr (FP8) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (t < ntiles) stg.write8(stage(t), raw[t]);
+    raw[1] = Raw8{};  // no longer live
+  }
   barrier_lds();
   if (2 < ntiles) {
-    stg.template copy_part<0, P>(item, stage(2), c_ptr, 2);
+    if constexpr (FP8)
+      stg.load8(item, c_ptr, 2, raw[0]);
+    else
+      stg.template copy_part<0, P>(item, stage(2), c_ptr, 2);
     advance();
   }
   if (0 < wave_kmax) qk(stage(0), s0);
@@ -939,7 +1051,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
     for (int t = 0; t < kStages; ++t) {
       const int it = it0 + t;
       if (it >= ntiles) break;
-      tile_iter(it, stage(t), stage(t + 1), stage(t + 3));
+      tile_iter(it, stage(t), stage(t + 1), stage(t + 3), stage(t + 2));
     }
   }
 
@@ -949,6 +1061,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   if (next.valid) {
     item_fetch_q<D>(p, next, qop);
     if constexpr (STORE) slot = item_fetch_slot(p, next);
+    if constexpr (FP8) item_fetch_tiles<KV, D>(p, smem_all, next, raw);
   }
   if constexpr (STORE) {
     if (rows_in_ring(item)) item_store_rows<D>(p, item, smem_all, s_slot);
@@ -957,10 +1070,12 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   if constexpr (SPLIT) {
     if (item.split_slot >= 0 && !merge_key_halves<D>(p, smem_all, item.split_slot, acc, m_run, l)) return;
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l > 0.f ? (FP8 ? p.v_scale[kvh] : 1.f) / l : 0.f;
   barrier_lds();  // every wave is done with the ring
   // stages 0 and 1 take the next item's first tiles
-  if (next.valid) item_fetch_tiles<PAGED, D>(p, smem_all, next);
+  if constexpr (!FP8) {
+    if (next.valid) item_fetch_tiles<KV, D>(p, smem_all, next, raw);
+  }
   // A work-queue grid claims the item after `next` here, one item ahead; the
   // caller reads the result after its own barrier, once the epilogue has run.
   if (claim_ctr != nullptr && next.valid && threadIdx.x == 0) claim = atomicAdd(claim_ctr, 1u);
@@ -999,7 +1114,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // on the same XCD (and its L2) whenever gridDim.x is a multiple of 8.  Tiles
 // past a sequence's end exit at once.  Used when the persistent grid's tables
 // would not fit its LDS.
-template <bool PAGED, int D, bool STORE>
+template <int KV, int D, bool STORE>
 __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
   if constexpr (STORE) {
@@ -1024,18 +1139,19 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillPara
   }
   ItemDesc it = item_desc(p, p.cu_q, p.cu_k, s, kvh, tile);
   if (!it.valid) return;
-  if (pair >= 0) key_half<PAGED>(p, it, half, pair * p.num_kv_heads + kvh);
+  if (pair >= 0) key_half<KV != kKvPacked>(p, it, half, pair * p.num_kv_heads + kvh);
   __shared__ int s_slot[STORE ? kRows : 1];
   int slot = -1;
   if constexpr (STORE) store_rows_ahead<D>(p, it);
   bf16x8 qop[D / 16];
   item_fetch_q<D>(p, it, qop);
-  item_fetch_tiles<PAGED, D>(p, smem_all, it);
+  Raw8 raw[2] = {};
+  item_fetch_tiles<KV, D>(p, smem_all, it, raw);
   if constexpr (STORE) slot = item_fetch_slot(p, it);
   ItemDesc none{};
   none.valid = false;
   uint32_t unused = 0;
-  prefill_run<PAGED, D, true, STORE>(p, smem_all, it, qop, none, nullptr, unused, s_slot, slot);
+  prefill_run<KV, D, true, STORE>(p, smem_all, it, qop, none, nullptr, unused, s_slot, slot, raw);
 }
 
 // Persistent grid: one workgroup per CU walks the real work items.
@@ -1087,7 +1203,7 @@ __device__ __forceinline__ int find_seq(const int* s_ntq, int S, int t, int rank
   return -1;
 }
 
-template <bool PAGED, int D, bool QUEUE, bool STORE>
+template <int KV, int D, bool QUEUE, bool STORE>
 __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
   __shared__ int s_ntq[kPersistMaxSeqs];           // query tiles of each sequence
@@ -1200,7 +1316,8 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
   bf16x8 qop[D / 16];
   int slot = -1;
   item_fetch_q<D>(p, cur, qop);
-  item_fetch_tiles<PAGED, D>(p, smem_all, cur);
+  Raw8 raw[2] = {};
+  item_fetch_tiles<KV, D>(p, smem_all, cur, raw);
   if constexpr (STORE) slot = item_fetch_slot(p, cur);
   for (int round = 1;; ++round) {
     // the next item is located (from the LDS tables) while this one's
@@ -1217,7 +1334,7 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
       nxt = desc_of(item64 < total ? static_cast<int>(item64) : total);
     }
     if constexpr (STORE) store_rows_ahead<D>(p, cur);
-    prefill_run<PAGED, D, false, STORE>(p, smem_all, cur, qop, nxt, claim_ctr, claim, s_slot, slot);
+    prefill_run<KV, D, false, STORE>(p, smem_all, cur, qop, nxt, claim_ctr, claim, s_slot, slot, raw);
     if (!nxt.valid) break;
     cur = nxt;
   }
@@ -1294,15 +1411,16 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   } while (0)
     if (fuse) {
       if (p.head_dim == 64)
-        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<false, 64, true, true>), grid, dim3(kThreads), 0, stream, p);
+        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<kKvPacked, 64, true, true>), grid, dim3(kThreads), 0, stream, p);
       else
-        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<false, 128, true, true>), grid, dim3(kThreads), 0, stream, p);
+        hipLaunchKernelGGL((varlen_prefill_persistent_kernel<kKvPacked, 128, true, true>), grid, dim3(kThreads), 0, stream, p);
     } else if (p.head_dim == 64) {
-      if (p.block_table) NVA_PERSIST(true, 64);
-      else NVA_PERSIST(false, 64);
+      if (p.block_table) NVA_PERSIST(kKvPaged, 64);
+      else NVA_PERSIST(kKvPacked, 64);
     } else {
-      if (p.block_table) NVA_PERSIST(true, 128);
-      else NVA_PERSIST(false, 128);
+      if (p.k_scale) NVA_PERSIST(kKvFp8, 128);
+      else if (p.block_table) NVA_PERSIST(kKvPaged, 128);
+      else NVA_PERSIST(kKvPacked, 128);
     }
 #undef NVA_PERSIST
     return hipGetLastError();
@@ -1329,13 +1447,14 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
 #define NVA_DIRECT(PG, DD, ST) \
   hipLaunchKernelGGL((varlen_prefill_kernel<PG, DD, ST>), grid, dim3(kThreads), 0, stream, p)
   if (p.head_dim == 64) {
-    if (p.block_table) NVA_DIRECT(true, 64, false);
-    else if (fuse) NVA_DIRECT(false, 64, true);
-    else NVA_DIRECT(false, 64, false);
+    if (p.block_table) NVA_DIRECT(kKvPaged, 64, false);
+    else if (fuse) NVA_DIRECT(kKvPacked, 64, true);
+    else NVA_DIRECT(kKvPacked, 64, false);
   } else {
-    if (p.block_table) NVA_DIRECT(true, 128, false);
-    else if (fuse) NVA_DIRECT(false, 128, true);
-    else NVA_DIRECT(false, 128, false);
+    if (p.k_scale) NVA_DIRECT(kKvFp8, 128, false);
+    else if (p.block_table) NVA_DIRECT(kKvPaged, 128, false);
+    else if (fuse) NVA_DIRECT(kKvPacked, 128, true);
+    else NVA_DIRECT(kKvPacked, 128, false);
   }
 #undef NVA_DIRECT
   return hipGetLastError();

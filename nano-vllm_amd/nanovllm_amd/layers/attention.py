@@ -14,8 +14,8 @@ names and argument meaning, backed by the gfx950 HIP library through its C ABI:
 Extension (not in the reference): an fp8 e4m3fn KV cache.  A module whose
 k_cache/v_cache are torch.float8_e4m3fn tensors must also carry k_scale/v_scale
 (float32, one per kv head; engine/kv_cache.allocate_kv_cache owns and binds
-them); store_kvcache then quantises x / scale, decode dequantises on the fly and a
-prefix-cached prefill gathers the pages into dequantised packed rows first.  A
+them); store_kvcache then quantises x / scale, decode and a prefix-cached prefill
+dequantise on the fly (a long prefill gathers the pages into packed rows first).  A
 prefill without a cached prefix reads the fresh bf16 k/v, as in the reference.
 
 Every launch goes to torch's current stream, nothing synchronises and the only
@@ -183,13 +183,29 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
     block_table is given (attention.py:67-73).  q (total_q, nh, d) -> (total_q, nh, d).
 
     Extension: paged caches in fp8 e4m3fn (with k_scale/v_scale, one float32 per
-    kv head) are first gathered into packed bf16 rows, dequantised
-    (nva_gather_kv), and the packed prefill runs on those.  That needs
+    kv head) are converted as the kernel stages them (nva_prefill_fp8), or, at other
+    head dims than 128, block sizes not a multiple of 64 and over _FP8_IN_PLACE_TOKENS
+    new tokens a sequence, first gathered into packed bf16 rows, dequantised
+    (nva_gather_kv), on which the packed prefill runs.  That needs
     cu_seqlens_k[s+1] - cu_seqlens_k[s] <= max_seqlen_k, as flash-attn does."""
     qa, kv, pages, rest, (out, *_rows) = _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k,
                                                        softmax_scale, causal, block_table, k_scale, v_scale)
-    _capi.check(_capi.load().nva_prefill(*qa, *kv, *pages, *rest))
+    if pages[0] is not None and k.dtype != _BF16:
+        k_ptr, _, v_ptr, _ = kv
+        _capi.check(_capi.load().nva_prefill_fp8(*qa, k_ptr, v_ptr, _ptr(k_scale), _ptr(v_scale), *pages, *rest))
+    else:
+        _capi.check(_capi.load().nva_prefill(*qa, *kv, *pages, *rest))
     return out
+
+
+# An fp8 prefill of up to this many new tokens per sequence reads the pages itself.  It then
+# converts a key tile once per query tile that sees it, ~3% of the loop's time, where the
+# gather converts each key once but writes it and reads it back at twice the bytes.  Heads
+# 16/8 and 32/8, gather + prefill against in place: 16 sequences of 20 tokens after 2048
+# cached ones 77 -> 36 us, 8 of 512 after 1024 67 -> 52 and 109 -> 94, 1 of 4096 after 2048
+# 174 -> 171 and 253 -> 247, 1 of 8192 after 8192 699 -> 705 and 1370 -> 1385 (heads 64/8,
+# the last two: 490 -> 488, 2686 -> 2735).
+_FP8_IN_PLACE_TOKENS = 4096
 
 
 def _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_k, softmax_scale, causal,
@@ -231,7 +247,8 @@ def _prefill_args(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu_seqlens_
         _check_scales(code, k_scale, v_scale, nkv, k.device)
         k_row = v_row = nkv * d
         bt_ptr, bt_stride, max_blocks = block_table.data_ptr(), block_table.stride(0), block_table.shape[1]
-        if code == _capi.NVA_DTYPE_FP8_E4M3:
+        if code == _capi.NVA_DTYPE_FP8_E4M3 and not (
+                d == 128 and block_size % 64 == 0 and int(max_seqlen_q) <= _FP8_IN_PLACE_TOKENS):
             # dequantise each sequence's pages into packed rows, then the packed prefill
             _check_device(q.device, k=k, v=v, cu_seqlens_k=cu_seqlens_k, block_table=block_table,
                           k_scale=k_scale, v_scale=v_scale)

@@ -192,3 +192,64 @@ def test_gather_kv_matches_oracle(dev, fp8):
                     x[j] = 0
             x = x.reshape(-1, 8, 128)[:n]
             assert np.array_equal(f32(packed[c[s]:c[s] + n]), x), f"{name} seq {s}"
+
+
+def _fp8_prefill_case(dev, lens, nh, nkv, d, bs, prefix, seed):
+    """A prefix-cached prefill over an fp8 cache whose pages already hold the fresh keys, and
+    the same case over the dequantised float32 cache for the oracle."""
+    from types import SimpleNamespace
+    from nanovllm_amd import workloads as W
+    blocks = sum(-(-(n + p) // bs) for n, p in zip(lens, prefix)) + 1
+    c = W.make_prefill_case(lens, nh, nkv, blocks, prefix_len=prefix, block_size=bs, head_dim=d, seed=seed,
+                            bulk_device=dev, shared_prefix=False)
+    c.k_cache, ks = W.quantize_cache_fp8(c.k_cache)
+    c.v_cache, vs = W.quantize_cache_fp8(c.v_cache)
+    deq = [torch.from_numpy(O.e4m3fn_to_f32(bits8(t)) * f32(s)[None, None, :, None])
+           for t, s in ((c.k_cache, ks), (c.v_cache, vs))]
+    ref = SimpleNamespace(**{**vars(c), "k_cache": deq[0], "v_cache": deq[1]})
+    return c, ks, vs, ref
+
+
+def _fp8_prefill(c, ks, vs):
+    import nanovllm_amd as nva
+    o = nva.flash_attn_varlen_func(c.q, c.k_cache, c.v_cache, c.max_seqlen_q, c.cu_seqlens_q, c.max_seqlen_k,
+                                   c.cu_seqlens_k, c.scale, block_table=c.block_tables, k_scale=ks, v_scale=vs)
+    torch.cuda.synchronize()
+    return f32(o)
+
+
+@pytest.mark.parametrize("nh,nkv", [(16, 8), (7, 1), (32, 2)])
+@pytest.mark.parametrize("bs", [64, 128, 256, 512])
+@pytest.mark.parametrize("shape", ["tile edges", "halves", "persistent"])
+def test_fp8_pages_converted_in_place(dev, nh, nkv, bs, shape):
+    """The prefill that converts fp8 pages as it stages them, at key counts around its 64-key
+    tiles and pages, on the direct grid, with key halves and on the persistent grid.  The
+    codes are exact in bf16 and the scales are applied in float32, so the bf16 bar holds
+    against the oracle on the dequantised cache."""
+    from _helpers import prefill_reference
+    lens, prefix = {"tile edges": ([1, 63, 64, 65, 128, 2], [bs, 0, bs, 2 * bs, 0, 3 * bs]),
+                    "halves": ([700, 30], [2 * bs, bs]),
+                    "persistent": ([130, 1, 257, 64] * 24, [bs, 0, 2 * bs, bs] * 24)}[shape]
+    c, ks, vs, ref = _fp8_prefill_case(dev, lens, nh, nkv, 128, bs, prefix, seed=bs + nh)
+    seqs = list(range(len(lens)))[-8:] + [0]
+    want = prefill_reference(ref, seqs)
+    cu = c.cu_seqlens_q.cpu().tolist()
+    for _ in range(2):
+        got = _fp8_prefill(c, ks, vs)
+        got = np.concatenate([got[cu[s]:cu[s + 1]] for s in seqs])
+        assert_attn_close(got, want, what=f"fp8 in place {shape} bs={bs}")
+
+
+@pytest.mark.parametrize("d,bs,limit", [(64, 64, None), (128, 96, None), (128, 256, 100)])
+def test_fp8_prefill_through_the_gather(dev, monkeypatch, d, bs, limit):
+    """Head dim 64, a block size not a multiple of 64 and more new tokens than the in-place limit
+    go through nva_gather_kv, whose rounding of the dequantised rows is inside the fp8 bar."""
+    from _helpers import prefill_reference
+    from nanovllm_amd.layers import attention as A
+    if limit:
+        monkeypatch.setattr(A, "_FP8_IN_PLACE_TOKENS", limit)
+    A._GATHER_BUFFERS.clear()
+    c, ks, vs, ref = _fp8_prefill_case(dev, [70, 1, 200], 8, 2, d, bs, [bs, 0, 2 * bs], seed=d + bs)
+    assert_attn_close(_fp8_prefill(c, ks, vs), prefill_reference(ref), max_abs=FP8_MAX_ABS, mean_abs=FP8_MAX_ABS,
+                      what="fp8 gather")
+    assert A._GATHER_BUFFERS
