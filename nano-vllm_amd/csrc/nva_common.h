@@ -112,9 +112,35 @@ __device__ __forceinline__ uint32_t f32_to_e4m3fn(float x) {
 }
 
 // Eight bf16 values (16 bytes, element e in bits 16 (e % 2) of word e / 2)
-// divided by `scale`, as eight e4m3fn codes (8 bytes, code e in byte e).
+// divided by `scale`, as eight e4m3fn codes (8 bytes, code e in byte e): bit for bit
+// f32_to_e4m3fn(x / scale) with an IEEE division.
+// For ordinary scales the quotient is x * r refined once by its exact remainder (r = 1 /
+// scale correctly rounded: Markstein's correctly rounded quotient; where the remainder
+// underflows, the quotient is far below the smallest code) and the hardware conversion,
+// which rounds as f32_to_e4m3fn does: about 7 instructions an element against 30.  The
+// sign is x's also for zeros, and NaN and overflow reach the conversion as infinities, which
+// it turns into 0x7f with the sign (a NaN's sign it would lose).  Equality was checked
+// for every bf16 x over 10^5 scales of 2^-30..2^30 and 10^5 of any bits.
 __device__ __forceinline__ u32x2 bf16x8_to_e4m3fn(u32x4 w, float scale) {
   u32x2 out;
+  if (scale > 0x1p-60f && scale < 0x1p60f) {
+    const float r = 1.f / scale;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float q[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t word = w[2 * h + (e >> 1)];
+        const float x = __builtin_bit_cast(float, (e & 1) ? word & 0xffff0000u : word << 16);
+        const float q0 = x * r;
+        const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, scale, x), r, q0);
+        q[e] = __builtin_copysignf(__builtin_fminf(__builtin_fabsf(q1), __builtin_huge_valf()), x);
+      }
+      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+      out[h] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true));
+    }
+    return out;
+  }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     uint32_t packed = 0;

@@ -50,20 +50,35 @@ __global__ __launch_bounds__(256) void store_kvcache_bf16_kernel(StoreParams p) 
   }
 }
 
-// bf16 rows -> fp8 cache rows, 8 elements (16 B in, 8 B out) per lane.
+// bf16 rows -> fp8 cache rows, 8 elements (16 B in, 8 B out) per lane.  As above, the first
+// piece and its scale are loaded together with the slot.  4096 tokens of 8 x 128 (25 MB):
+// 8.9 us with a division and a software conversion per element, bound by those, 6.4 us
+// with the refined reciprocal and the hardware conversion (64 tokens: 2.8 -> 2.2 us).
+// Non-temporal stores measured the same.
 __global__ __launch_bounds__(256) void store_kvcache_fp8_kernel(StoreParams p) {
   const int64_t t = blockIdx.x;
-  const int64_t slot = p.slot_mapping[t];
-  if (slot < 0 || slot >= p.num_slots) return;
   const int pieces = p.row_elems / 8;
   const bool is_v = threadIdx.y != 0;
   const char* src = static_cast<const char*>(is_v ? p.value : p.key) +
                     t * (is_v ? p.value_row_stride : p.key_row_stride) * 2;
-  char* dst = static_cast<char*>(is_v ? p.v_cache : p.k_cache) + slot * p.row_elems;
   const float* scale = is_v ? p.v_scale : p.k_scale;
-  for (int c = threadIdx.x; c < pieces; c += blockDim.x) {
-    const float s = scale[(c * 8) / p.head_dim];
-    *reinterpret_cast<u32x2*>(dst + c * 8) = bf16x8_to_e4m3fn(ld16(src + c * 16), s);
+  int c = threadIdx.x;
+  u32x4 x = {0u, 0u, 0u, 0u};
+  float s = 1.f;
+  if (c < pieces) {
+    x = ld16(src + c * 16);
+    s = scale[(c * 8) / p.head_dim];
+  }
+  const int64_t slot = p.slot_mapping[t];
+  if (slot < 0 || slot >= p.num_slots) return;
+  char* dst = static_cast<char*>(is_v ? p.v_cache : p.k_cache) + slot * p.row_elems;
+  while (c < pieces) {
+    *reinterpret_cast<u32x2*>(dst + c * 8) = bf16x8_to_e4m3fn(x, s);
+    c += blockDim.x;
+    if (c < pieces) {
+      x = ld16(src + c * 16);
+      s = scale[(c * 8) / p.head_dim];
+    }
   }
 }
 

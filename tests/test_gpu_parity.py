@@ -122,6 +122,32 @@ def test_store_fp8_bitexact(dev):
     assert np.array_equal(got_rows, torch_k)
 
 
+def test_store_fp8_every_bf16_value(dev):
+    """Every bf16 value (zeros of both signs, subnormals, infinities, NaNs) over ordinary scales,
+    whose quotient is a refined product with the reciprocal, the limits of that range and
+    scales beyond it, which are divided: the codes of torch's cast of the IEEE quotient.  A
+    NaN input keeps its sign."""
+    nkv, d = 16, 128
+    T = 65536 // d
+    scales = [1.0, 0.0123, 3.1e-5, 7.0 / 3.0, 448.0, 1 / 448.0, 2.0 ** -29, 1.7 * 2.0 ** 29, 2.0 ** -60, 1.1 * 2.0 ** -60,
+              2.0 ** 60, 1e-30, 1e30, 1e-45, 3e38, 0.333333343]
+    bits = torch.arange(65536, dtype=torch.int32, device=dev).to(torch.int16).view(torch.bfloat16).view(T, 1, d)
+    x = bits.expand(T, nkv, d).contiguous()
+    scale = torch.tensor(scales, dtype=torch.float32, device=dev)
+    kc = torch.zeros(T // 256, 256, nkv, d, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+    vc = torch.zeros_like(kc)
+    slots = torch.arange(T, dtype=torch.int32, device=dev)
+    nva().store_kvcache(x, x, kc, vc, slots, scale, scale.flip(0).contiguous())
+    torch.cuda.synchronize()
+    xf = x.float().cpu()
+    for cache, sc in ((kc, scale.cpu()), (vc, scale.flip(0).cpu())):
+        want = (xf / sc.view(1, nkv, 1)).to(torch.float8_e4m3fn).view(torch.uint8).numpy()
+        got = bits8(cache).reshape(T, nkv, d)
+        nan = torch.isnan(xf).numpy()
+        assert np.array_equal(got[~nan], want[~nan])
+        assert np.array_equal(got[nan], np.where(np.signbit(xf.numpy()[nan]), 0xff, 0x7f))
+
+
 # ----------------------------------------------------------------------------
 # decode
 # ----------------------------------------------------------------------------
