@@ -4,7 +4,9 @@ Usage:  python nano-vllm_amd/build.py [--jobs N] [--verbose]
 
 Every .hip file under csrc/ is compiled to an object under _build/ and the
 objects are linked into nanovllm_amd/_lib/libnva_attn.so, which the Python
-host side loads with ctypes.  No GPU is needed to build.
+host side loads with ctypes.  csrc/host/nva_host.cpp becomes the CPython module
+_nva_host.so beside it (g++ against torch's headers and libraries).  No GPU is
+needed to build.
 """
 from __future__ import annotations
 
@@ -14,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
@@ -22,6 +25,8 @@ INCLUDE = HERE.parent / "include"
 BUILD = HERE / "_build"
 LIB_DIR = HERE / "nanovllm_amd" / "_lib"
 LIB = LIB_DIR / "libnva_attn.so"
+HOST_SRC = CSRC / "host" / "nva_host.cpp"
+HOST_LIB = LIB_DIR / "_nva_host.so"
 ARCH = "gfx950"
 
 # Packed fp32 VALU ops are disabled: the kernels are written with scalar and
@@ -72,6 +77,26 @@ def _compile(src: Path, verbose: bool) -> Path:
     return obj
 
 
+def _build_host(verbose: bool) -> None:
+    """The host module, linked against the installed torch (its ABI)."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    tmp = HOST_LIB.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{INCLUDE}", "-isystem", str(root / "include"),
+           "-isystem", str(root / "include" / "torch" / "csrc" / "api" / "include"), "-isystem", str(rocm / "include"),
+           "-isystem", sysconfig.get_paths()["include"], str(HOST_SRC), "-o", str(tmp), f"-L{root / 'lib'}",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SRC.name}:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_LIB)
+
+
 def build(jobs: int = 4, verbose: bool = False) -> Path:
     BUILD.mkdir(exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
@@ -79,7 +104,9 @@ def build(jobs: int = 4, verbose: bool = False) -> Path:
     if not sources:
         raise RuntimeError(f"no .hip sources under {CSRC}")
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        host = ex.submit(_build_host, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), sources))
+        host.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:

@@ -6,6 +6,7 @@ if it is missing or fails to load, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -163,6 +164,28 @@ def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:
         if path is None:
             _lib = lib
         return lib
+
+
+HOST_PATH = LIB_PATH.parent / "_nva_host.so"
+# the entry points that the host module calls, in the order of its bind()
+_HOST_ENTRIES = ("nva_store_kvcache", "nva_prefill", "nva_prefill_fp8", "nva_store_prefill",
+                 "nva_decode_workspace_bytes", "nva_decode", "nva_store_decode", "nva_qk_norm_rope")
+_host = None
+
+
+def host():
+    """The native form of the per-step calls (csrc/host/nva_host.cpp), bound to the loaded library."""
+    global _host
+    if _host is None:
+        lib = load()
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is not built: run `python nano-vllm_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("_nva_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES))
+        _host = mod
+    return _host
 
 
 def check(status: int) -> None:

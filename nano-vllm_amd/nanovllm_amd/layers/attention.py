@@ -407,10 +407,19 @@ class Attention(nn.Module):
         self.fuse_decode_store = False
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
+        context = get_context()
+        # the ordinary form of the call in native code; None: anything else, below
+        o = _capi.host().attention(
+            q, k, v, self.k_cache, self.v_cache, self.k_scale, self.v_scale, self.num_heads, self.num_kv_heads,
+            self.head_dim, self.scale, self.fuse_decode_store, context.is_prefill, context.cu_seqlens_q,
+            context.cu_seqlens_k, context.max_seqlen_q, context.max_seqlen_k, context.slot_mapping,
+            context.context_lens, context.block_tables, _PREFILL_WORKSPACES, _FP8_IN_PLACE_TOKENS)
+        return o if o is not None else self._forward_general(q, k, v, context)
+
+    def _forward_general(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, context):
         q = q.view(-1, self.num_heads, self.head_dim)
         k = k.view(-1, self.num_kv_heads, self.head_dim)
         v = v.view(-1, self.num_kv_heads, self.head_dim)
-        context = get_context()
         k_cache, v_cache = self.k_cache, self.v_cache
         bound = k_cache.numel() and v_cache.numel()
         if not context.is_prefill and bound and self.fuse_decode_store:  # store and attention as one call

@@ -50,6 +50,11 @@ def qk_norm_rope(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, cos_
                  eps: float = 1e-6, inplace: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """Returns (q, k) after the per-head RMSNorm (when weights are given) and the
     rotary embedding, in q's and k's shapes.  inplace=True writes into q and k."""
+    if not inplace:  # the ordinary form in native code; None: anything else
+        pair = _capi.host().qk_norm_rope(positions, q, k, cos_sin_cache, num_heads, num_kv_heads, head_dim,
+                                         q_norm_weight, k_norm_weight, eps)
+        if pair is not None:
+            return pair
     T, q_rs = _rows(q, num_heads, head_dim, "q")
     Tk, k_rs = _rows(k, num_kv_heads, head_dim, "k")
     if Tk != T or positions.shape != (T,) or positions.dtype != torch.int64:

@@ -1,0 +1,218 @@
+"""The native form of Attention.forward and qk_norm_rope (csrc/host/nva_host.cpp): bit-identical
+to the general Python path over the forms it takes, None (and so the general path) for the
+others."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    from nanovllm_amd import _capi
+    _capi.load()
+    return torch.device("cuda:0")
+
+
+class _Off:
+    """A host module that takes nothing."""
+
+    @staticmethod
+    def attention(*args):
+        return None
+
+    @staticmethod
+    def qk_norm_rope(*args):
+        return None
+
+
+class _Spy:
+    def __init__(self, real):
+        self.real, self.taken = real, 0
+
+    def attention(self, *args):
+        o = self.real.attention(*args)
+        self.taken += o is not None
+        return o
+
+    def qk_norm_rope(self, *args):
+        o = self.real.qk_norm_rope(*args)
+        self.taken += o is not None
+        return o
+
+
+def _layer(c, k_cache, v_cache, scales=(None, None)):
+    import nanovllm_amd as nva
+    layer = nva.Attention(c.num_heads, c.head_dim, c.scale, c.num_kv_heads)
+    layer.k_cache, layer.v_cache = k_cache, v_cache
+    layer.k_scale, layer.v_scale = scales
+    return layer
+
+
+def _both(monkeypatch, run):
+    """run() through the general path and through the native one; each returns its tensors."""
+    from nanovllm_amd import _capi
+    real = _capi.host()
+    with monkeypatch.context() as m:
+        m.setattr(_capi, "_host", _Off)
+        want = run()
+    spy = _Spy(real)
+    with monkeypatch.context() as m:
+        m.setattr(_capi, "_host", spy)
+        got = run()
+    torch.cuda.synchronize()
+    return want, got, spy.taken
+
+
+def _same(want, got):
+    for a, b in zip(want, got):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["2d", "3d", "strided"])
+@pytest.mark.parametrize("prefix", [0, 256])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_prefill_equals_the_general_path(dev, monkeypatch, form, prefix, fp8):
+    import nanovllm_amd as nva
+    from nanovllm_amd import workloads as W
+    c = W.make_prefill_case([30, 1, 100], 16, 8, 12, prefix_len=prefix, seed=3, bulk_device=dev)
+    scales = (None, None)
+    if fp8:
+        c.k_cache, ks = W.quantize_cache_fp8(c.k_cache, extra=c.k)
+        c.v_cache, vs = W.quantize_cache_fp8(c.v_cache, extra=c.v)
+        scales = (ks, vs)
+    q, k, v = c.q, c.k, c.v
+    if form == "2d":
+        q, k = q.view(-1, 2048), k.view(-1, 1024)
+    elif form == "strided":
+        qkv = torch.cat([t.reshape(t.shape[0], -1) for t in (q, k, v)], dim=1)
+        q, k, v = qkv[:, :2048], qkv[:, 2048:3072], qkv[:, 3072:]
+
+    def run():
+        layer = _layer(c, c.k_cache.clone(), c.v_cache.clone(), scales)
+        nva.set_context(True, c.cu_seqlens_q, c.cu_seqlens_k, c.max_seqlen_q, c.max_seqlen_k, c.slot_mapping, None,
+                        c.block_tables)
+        o = layer(q, k, v)
+        nva.reset_context()
+        return o, layer.k_cache, layer.v_cache
+    run()  # the stream's workspace
+    want, got, taken = _both(monkeypatch, run)
+    _same(want, got)
+    assert taken == 1
+
+
+def _decode_inputs(dev, B, nh, nkv, d, fp8, seed):
+    from nanovllm_amd import workloads as W
+    base = [1, 33, 0, 256, 257, 700, 31, 32, 64, 900]
+    lens = [base[i % len(base)] for i in range(B)]
+    return W.make_decode_case(B, nh, nkv, 0, 0, 5 * B + 2, head_dim=d, fp8=fp8, seed=seed, bulk_device=dev, lengths=lens,
+                              table_width=4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slots", ["own", "rolled", "inside", "foreign", "padding", "out of range"])
+@pytest.mark.parametrize("B,nh,nkv,d,fp8", [(1, 16, 8, 128, False), (10, 16, 8, 128, False), (10, 64, 8, 128, True),
+                                            (32, 16, 8, 128, False), (100, 14, 2, 64, False), (200, 4, 1, 128, False),
+                                            (64, 16, 8, 128, False)])
+def test_decode_equals_store_then_decode(dev, monkeypatch, slots, B, nh, nkv, d, fp8):
+    """Store, then decode, for any slots: spread mode (batch x kv heads up to 256) and, last,
+    the balanced mode."""
+    import nanovllm_amd as nva
+    c = _decode_inputs(dev, B, nh, nkv, d, fp8, seed=B)
+    s = c.slot_mapping
+    live = [b for b, n in enumerate(c.lengths) if n > 0]
+    if slots == "padding" and B == 1:
+        pytest.skip("one live row")
+    if slots == "rolled":  # row b goes to another sequence's last key
+        s[live] = s[live].roll(1)
+    elif slots == "inside":  # row b goes to the middle of its own context
+        for b in live:
+            n = c.lengths[b] // 2
+            s[b] = int(c.block_tables[b, n // 256]) * 256 + n % 256
+    elif slots == "foreign":  # row b goes to the first key of the sequence after it
+        s[live] = (c.block_tables[live, 0] * 256).roll(-1)
+    elif slots == "padding":  # rows without keys go to slots that live sequences read
+        # (of more than one key: the row of a one-key sequence goes to that very slot, and which
+        # of two rows a slot keeps is not defined by the store either)
+        empty = [b for b, n in enumerate(c.lengths) if n == 0]
+        longer = [b for b in live if c.lengths[b] > 1]
+        for i, b in enumerate(empty):
+            s[b] = int(c.block_tables[longer[i % len(longer)], 0]) * 256
+    elif slots == "out of range":
+        s[::2] = -1
+        s[1::2] = c.k_cache.shape[0] * 256
+
+    def run():
+        layer = _layer(c, c.k_cache.clone(), c.v_cache.clone(), (c.k_scale, c.v_scale))
+        nva.set_context(False, slot_mapping=s, context_lens=c.context_lens, block_tables=c.block_tables)
+        o = layer(c.q, c.k_new, c.v_new)
+        nva.reset_context()
+        return o, layer.k_cache, layer.v_cache
+    want, got, taken = _both(monkeypatch, run)
+    assert taken == 1
+    _same(want, got)
+
+
+@pytest.mark.gpu
+def test_producer_equals_the_general_path(dev, monkeypatch):
+    from nanovllm_amd import workloads as W
+    from nanovllm_amd.layers.qk_norm_rope import qk_norm_rope
+    for nh, nkv, d, norm in ((16, 8, 128, True), (14, 2, 64, False)):
+        c = W.make_producer_case(19, nh, nkv, head_dim=d, norm=norm, seed=2, device=dev)
+        for q, k in ((c.q, c.k), (c.qkv[:, :nh * d], c.qkv[:, nh * d:(nh + nkv) * d])):
+            want, got, taken = _both(monkeypatch, lambda: qk_norm_rope(
+                c.positions, q, k, c.cos_sin_cache, nh, nkv, d, c.q_norm_weight, c.k_norm_weight))
+            _same(want, got)
+            assert taken == 1
+
+
+@pytest.mark.gpu
+def test_other_forms_are_left_to_the_general_path(dev):
+    """Wrapped tensors, active modes and forms that the general path converts or refuses."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from nanovllm_amd import _capi
+    c = _decode_inputs(dev, 10, 16, 8, 128, False, seed=1)
+
+    def call(**kw):
+        a = dict(q=c.q, k=c.k_new, v=c.v_new, kc=c.k_cache, vc=c.v_cache, ks=None, vs=None, nh=16, nkv=8, d=128,
+                 scale=c.scale, fuse=False, pre=False, cq=None, ck=None, mq=0, mk=0, slots=c.slot_mapping,
+                 lens=c.context_lens, bt=c.block_tables, ws={}, lim=4096)
+        a.update(kw)
+        return _capi.host().attention(*a.values())
+
+    assert call() is not None
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    for kw in (dict(q=c.q.float()), dict(q=c.q.cpu()), dict(q=c.q.as_subclass(Sub)), dict(q=c.q[:, ::2]),
+               dict(q=c.q[:9]), dict(slots=c.slot_mapping.long()), dict(slots=c.slot_mapping.cpu()),
+               dict(lens=c.context_lens[:9]), dict(bt=c.block_tables.t()), dict(bt=None), dict(scale=1), dict(nh=True),
+               dict(kc=c.k_cache.transpose(0, 1)), dict(kc=c.k_cache.half()), dict(nh=12), dict(pre=1),
+               dict(pre=True, cq=c.context_lens, ck=c.context_lens), dict(kc=torch.tensor([]), vc=torch.tensor([]))):
+        assert call(**kw) is None, kw.keys()
+    with Mode():
+        assert call() is None
+    assert torch.func.vmap(lambda x: (call(q=x) is None) * x.sum())(c.q.unsqueeze(0)) is not None
+    seen = []
+    torch.func.vmap(lambda x: (seen.append(call(q=x)), x)[1])(c.q.unsqueeze(0))
+    assert seen == [None]
+
+
+def test_host_tensors_are_left_to_the_general_path():
+    from nanovllm_amd import _capi
+    x = torch.zeros(2, 8, 128, dtype=torch.bfloat16)
+    i = torch.zeros(2, dtype=torch.int32)
+    kc = torch.zeros(2, 256, 8, 128, dtype=torch.bfloat16)
+    host = _capi.host()
+    assert host.attention(x, x, x, kc, kc, None, None, 8, 8, 128, 0.1, False, False, None, None, 0, 0, i, i,
+                          torch.zeros(2, 1, dtype=torch.int32), {}, 4096) is None
+    assert host.attention() is None and host.qk_norm_rope() is None
+    assert host.qk_norm_rope(i.long(), x, x, torch.zeros(4, 128), 8, 8, 128, None, None, 1e-6) is None
