@@ -243,6 +243,26 @@ int nva_store_decode(const void* key, int64_t key_row_stride,
                      void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * nva_store_kvcache of the new rows, then nva_decode, with the results of the two calls for any
+ * slots (nva_store_decode without its conditions; same arguments).  In the spread mode the
+ * store runs inside the decode launch: a wave that reads the slot of another row of the step
+ * writes that row first.  Other plans launch the store before the decode, as do rows, queries
+ * or an output that lie inside a cache.
+ */
+int nva_store_then_decode(const void* key, int64_t key_row_stride,
+                          const void* value, int64_t value_row_stride,
+                          const int32_t* slot_mapping,
+                          const void* q, int64_t q_row_stride,
+                          void* k_cache, void* v_cache, int32_t kv_dtype,
+                          const float* k_scale, const float* v_scale, int64_t num_blocks,
+                          const int32_t* cache_seqlens, const int32_t* block_table,
+                          int64_t bt_row_stride, int32_t max_blocks_per_seq, int32_t block_size,
+                          int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                          float softmax_scale, int32_t num_splits,
+                          void* out, int64_t out_row_stride,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Gather each sequence's keys and values from the paged caches into packed bf16 rows:
  * key j of sequence s (block block_table[s*bt_row_stride + j/block_size], j < cu_seqlens_k[s+1] -
  * cu_seqlens_k[s]) goes to row cu_seqlens_k[s] + j of k_out / v_out.  An fp8 e4m3fn cache is

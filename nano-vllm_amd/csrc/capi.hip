@@ -382,7 +382,7 @@ int decode_impl(const void* q, int64_t q_row_stride, const void* k_cache, const 
                 int32_t batch, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float softmax_scale,
                 int32_t num_splits, void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes,
                 void* stream, int64_t scratch_max, void* (*get_scratch)(),
-                const nva::StoreParams* store = nullptr, int store_vec = 0) {
+                const nva::StoreParams* store = nullptr, int store_vec = 0, bool store_exact = false) {
   if (head_dim != 128 && head_dim != 64)
     return fail(NVA_ERR_UNSUPPORTED, "head_dim %d not supported (64 or 128)", head_dim);
   if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0)
@@ -479,12 +479,14 @@ int decode_impl(const void* q, int64_t q_row_stride, const void* k_cache, const 
     // bf16 cache, store inside their own launch (16-byte source pieces): the
     // rows of sequences with keys in the decode kernel, those of sequences
     // with none in the merge kernel that follows it.  Otherwise the store
-    // kernel runs first.
+    // kernel runs first.  store_exact: only the spread mode, whose few rows every
+    // wave can check against its keys.
     // (The fused kernels compare slots in 32 bits: pools below 2^31 slots.)
     const bool bf16_vec = kv_dtype == NVA_DTYPE_BF16 && store_vec == 16;
     const bool small_pool = num_blocks * block_size < (int64_t{1} << 31);
     if (small_pool && ((plan.spread > 1 && (kv_dtype == NVA_DTYPE_FP8_E4M3 || store_vec == 16)) ||
-                       (plan.balanced_ranges > 0 && bf16_vec))) {
+                       (plan.balanced_ranges > 0 && bf16_vec && !store_exact))) {
+      p.store_exact = store_exact ? 1 : 0;
       p.new_k = static_cast<const uint16_t*>(store->key);
       p.new_v = static_cast<const uint16_t*>(store->value);
       p.new_k_stride = store->key_row_stride;
@@ -532,6 +534,40 @@ int nva_store_decode(const void* key, int64_t key_row_stride, const void* value,
                      block_table, bt_row_stride, max_blocks_per_seq, block_size, batch, num_heads, num_kv_heads,
                      head_dim, softmax_scale, num_splits, out, out_row_stride, workspace, workspace_bytes, stream, 0,
                      nullptr, batch > 0 ? &sp : nullptr, vec);
+}
+
+int nva_store_then_decode(const void* key, int64_t key_row_stride, const void* value, int64_t value_row_stride,
+                          const int32_t* slot_mapping, const void* q, int64_t q_row_stride, void* k_cache, void* v_cache,
+                          int32_t kv_dtype, const float* k_scale, const float* v_scale, int64_t num_blocks,
+                          const int32_t* cache_seqlens, const int32_t* block_table, int64_t bt_row_stride,
+                          int32_t max_blocks_per_seq, int32_t block_size, int32_t batch, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t head_dim, float softmax_scale, int32_t num_splits, void* out,
+                          int64_t out_row_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (num_blocks <= 0 || block_size <= 0 || num_blocks > INT64_MAX / block_size)
+    return fail(NVA_ERR_INVALID_ARGUMENT, "num_blocks and block_size must be positive");
+  nva::StoreParams sp{};
+  int vec = 2;
+  const int rc = store_setup(key, key_row_stride, value, value_row_stride, k_cache, v_cache, num_blocks * block_size,
+                             slot_mapping, batch, num_kv_heads, head_dim, kv_dtype, k_scale, v_scale, sp, vec);
+  if (rc != NVA_OK) return rc;
+  // Rows or queries inside the caches, or an output there: the store has to be done first.
+  bool apart = batch == 0;
+  if (batch > 0 && num_heads > 0) {
+    const int64_t D = static_cast<int64_t>(num_kv_heads) * head_dim, qd = static_cast<int64_t>(num_heads) * head_dim;
+    const int64_t bytes = num_blocks * block_size * D * (kv_dtype == NVA_DTYPE_BF16 ? 2 : 1);
+    for (const void* c : {k_cache, v_cache})
+      apart = apart || rows_overlap(key, batch, key_row_stride, D, c, bytes) ||
+              rows_overlap(value, batch, value_row_stride, D, c, bytes) || rows_overlap(q, batch, q_row_stride, qd, c, bytes) ||
+              rows_overlap(out, batch, out_row_stride, qd, c, bytes);
+    if (apart) {
+      const hipError_t e = nva::launch_store_kvcache(sp, vec, static_cast<hipStream_t>(stream));
+      if (e != hipSuccess) return hip_status(e, "store_kvcache launch");
+    }
+  }
+  return decode_impl(q, q_row_stride, k_cache, v_cache, kv_dtype, k_scale, v_scale, num_blocks, cache_seqlens,
+                     block_table, bt_row_stride, max_blocks_per_seq, block_size, batch, num_heads, num_kv_heads,
+                     head_dim, softmax_scale, num_splits, out, out_row_stride, workspace, workspace_bytes, stream, 0,
+                     nullptr, apart ? nullptr : &sp, vec, true);
 }
 
 int64_t nva_decode_noalloc_max_workspace_bytes(void) { return kDecodeScratchBytes; }

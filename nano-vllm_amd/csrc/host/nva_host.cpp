@@ -4,7 +4,7 @@
 //
 // A small call is bound by the host: with the checks, tensor creations and ctypes
 // conversions in Python, a decode of one sequence took 30 us for 10 us of kernels; here
-// the whole call costs 16.5 us, little more than its three launches.
+// the whole call costs 10.2 us, little more than its two launches.
 //
 // Every function takes the ordinary form of its arguments -- plain dense GPU tensors of the
 // documented types, shapes and strides on one device, no dispatch or function mode -- and
@@ -34,6 +34,7 @@ struct Abi {
   decltype(&nva_decode_workspace_bytes) decode_workspace_bytes;
   decltype(&nva_decode) decode;
   decltype(&nva_store_decode) store_decode;
+  decltype(&nva_store_then_decode) store_then_decode;
   decltype(&nva_qk_norm_rope) qk_norm_rope;
 } abi{};
 bool bound = false;
@@ -178,8 +179,8 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* const wsp = ws_bytes > 0 ? ws.mutable_data_ptr() : nullptr;
     void *op = out.mutable_data_ptr(), *kp = kc->mutable_data_ptr(), *vp = vc->mutable_data_ptr();
     Py_BEGIN_ALLOW_THREADS
-    if (fuse) {
-      rc = abi.store_decode(
+    if (N == T) {
+      rc = (fuse ? abi.store_decode : abi.store_then_decode)(
           data<void>(k), k->stride(0), data<void>(v), v->stride(0), data<int32_t>(slots), data<void>(q), q->stride(0),
           kp, vp, code, data<float>(ks), data<float>(vs), num_blocks, data<int32_t>(lens), data<int32_t>(bt),
           bt->stride(0), static_cast<int32_t>(bt->size(1)), static_cast<int32_t>(block_size), static_cast<int32_t>(T),

@@ -62,6 +62,7 @@ struct DecodeParams {
   const int32_t* slot_mapping;
   float scale_log2;           // softmax_scale * log2(e)
   int32_t kv_fp8;             // 1: e4m3fn cache (k_scale / v_scale), 0: bf16
+  int32_t store_exact;        // spread mode: equal to store-then-decode for any slots
 };
 
 struct PrefillParams {

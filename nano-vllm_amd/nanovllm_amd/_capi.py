@@ -87,6 +87,17 @@ SIGNATURES = {
         _c_void_p, _i64,                   # out, out_row_stride
         _c_void_p, _i64, _c_void_p,        # workspace, workspace_bytes, stream
     ]),
+    "nva_store_then_decode": (_i32, [
+        _c_void_p, _i64, _c_void_p, _i64,  # key, key_row_stride, value, value_row_stride
+        _c_void_p,                         # slot_mapping
+        _c_void_p, _i64,                   # q, q_row_stride
+        _c_void_p, _c_void_p, _i32,        # k_cache, v_cache, kv_dtype
+        _c_void_p, _c_void_p, _i64,        # k_scale, v_scale, num_blocks
+        _c_void_p, _c_void_p, _i64, _i32, _i32,  # seqlens, block_table, bt_row_stride, max_blocks, block_size
+        _i32, _i32, _i32, _i32, _f32, _i32,  # batch, nh, nkv, head_dim, scale, num_splits
+        _c_void_p, _i64,                   # out, out_row_stride
+        _c_void_p, _i64, _c_void_p,        # workspace, workspace_bytes, stream
+    ]),
     "nva_decode": (_i32, [
         _c_void_p, _i64,                   # q, q_row_stride
         _c_void_p, _c_void_p, _i32,        # k_cache, v_cache, kv_dtype
@@ -169,7 +180,8 @@ def load(path: str | os.PathLike | None = None) -> ctypes.CDLL:
 HOST_PATH = LIB_PATH.parent / "_nva_host.so"
 # the entry points that the host module calls, in the order of its bind()
 _HOST_ENTRIES = ("nva_store_kvcache", "nva_prefill", "nva_prefill_fp8", "nva_store_prefill",
-                 "nva_decode_workspace_bytes", "nva_decode", "nva_store_decode", "nva_qk_norm_rope")
+                 "nva_decode_workspace_bytes", "nva_decode", "nva_store_decode", "nva_store_then_decode",
+                 "nva_qk_norm_rope")
 _host = None
 
 

@@ -1,6 +1,7 @@
 """The native form of Attention.forward and qk_norm_rope (csrc/host/nva_host.cpp): bit-identical
 to the general Python path over the forms it takes, None (and so the general path) for the
-others."""
+others, and the store inside a small batch's decode launch equal to store-then-decode for any
+slots."""
 from __future__ import annotations
 
 import pytest
@@ -118,8 +119,7 @@ def _decode_inputs(dev, B, nh, nkv, d, fp8, seed):
                                             (32, 16, 8, 128, False), (100, 14, 2, 64, False), (200, 4, 1, 128, False),
                                             (64, 16, 8, 128, False)])
 def test_decode_equals_store_then_decode(dev, monkeypatch, slots, B, nh, nkv, d, fp8):
-    """Store, then decode, for any slots: spread mode (batch x kv heads up to 256) and, last,
-    the balanced mode."""
+    """Spread mode (batch x kv heads up to 256) and, last, the balanced mode."""
     import nanovllm_amd as nva
     c = _decode_inputs(dev, B, nh, nkv, d, fp8, seed=B)
     s = c.slot_mapping
