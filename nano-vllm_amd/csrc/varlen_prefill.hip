@@ -93,30 +93,46 @@ __device__ __forceinline__ bf16x8 read_tr_pair(const char* p0, const char* p1) {
 
 }  // namespace
 
-// Per-lane constants of the staging of a tile: every wave moves P 1 KiB
-// pieces; lane `lane` of piece u carries key row `row[u]`, element offset
-// `col[u]` inside that row (K for waves 0..3, V for 4..7).
+// The thread index passes through an empty asm so that everything derived
+// from it (operand addresses, staging offsets) is formed where it is used:
+// hoisted out of the persistent kernel's item loop, those values would stay
+// live across items and push the register count past 256.
+__device__ __forceinline__ int laundered_tid() {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
+// Staging of a tile: every wave moves P 1 KiB pieces; lane `lane` of piece u of
+// wave w carries 16 bytes of key row `row`, from element `col` of that row (K for
+// waves 0..3, V for 4..7).
+template <int D>
+__device__ __forceinline__ void stage_piece(int w, int lane, int u, int& row, int& col) {
+  using Gm = Geom<D>;
+  const int off = (Gm::P * w + u) * 1024;
+  const int local = (off & (Gm::kTileBytes - 1)) + 16 * lane;
+  row = local / Gm::RB;
+  const int piece = (local >> 4) & (Gm::KP - 1);
+  col = off < Gm::kTileBytes ? (piece ^ Gm::k_swz(row)) * 8 : ((piece >> 1) ^ Gm::v_swz(row)) * 16 + (piece & 1) * 8;
+}
+
+// What a lane keeps of it: row, col and the byte offset of (row, col) from the tile's first
+// key.  (LEAN kernels form row and column again for a tile with keys missing, the item's
+// last, to save the registers.)
 template <int P>
 struct StageLane {
   int row[P];
   int col[P];
-  uint32_t off[P];  // byte offset of (row, col) from the tile's first key
+  uint32_t off[P];
 };
 
 template <int D>
 __device__ __forceinline__ StageLane<Geom<D>::P> stage_lane(int w, int lane, int64_t stride) {
-  using Gm = Geom<D>;
-  StageLane<Gm::P> d;
+  StageLane<Geom<D>::P> d;
 #pragma unroll
-  for (int u = 0; u < Gm::P; ++u) {
-    const int off = (Gm::P * w + u) * 1024;
-    const int local = (off & (Gm::kTileBytes - 1)) + 16 * lane;
-    const int row = local / Gm::RB;
-    const int piece = (local >> 4) & (Gm::KP - 1);
-    d.row[u] = row;
-    d.col[u] = off < Gm::kTileBytes ? (piece ^ Gm::k_swz(row)) * 8
-                                    : ((piece >> 1) ^ Gm::v_swz(row)) * 16 + (piece & 1) * 8;
-    d.off[u] = static_cast<uint32_t>((row * stride + d.col[u]) * 2);
+  for (int u = 0; u < Geom<D>::P; ++u) {
+    stage_piece<D>(w, lane, u, d.row[u], d.col[u]);
+    d.off[u] = static_cast<uint32_t>((d.row[u] * stride + d.col[u]) * 2);
   }
   return d;
 }
@@ -218,21 +234,26 @@ __device__ __forceinline__ void wait_vmem() {
 // Copy this wave's P KiB of one 64-key K/V tile (at `tile`, key kb) into the
 // stage whose K tile is at `st` (its V tile v_skip + tile bytes further on):
 // lane `lane` of piece u lands at (P w + u) KiB + 16 lane and carries the
-// swizzled (row, col) of StageLane.  Keys at or beyond kmax (only in the last
+// swizzled (row, col) of stage_piece.  Keys at or beyond kmax (only in the last
 // tile) are redirected to the tile's first key, a valid row whose scores the
 // masks remove.
-template <int P, int U0 = 0, int U1 = P>
-__device__ __forceinline__ void dma_tile(char* st, const char* tile, const StageLane<P>& d, int kb, int kmax, int w,
-                                         int v_skip) {
+template <int D, bool LEAN, int U0 = 0, int U1 = Geom<D>::P>
+__device__ __forceinline__ void dma_tile(char* st, const char* tile, const StageLane<Geom<D>::P>& d, int kb, int kmax,
+                                         int w, int v_skip) {
+  constexpr int P = Geom<D>::P;
   const uint32_t dst = lds_addr(st) + v_skip + P * w * 1024;
   if (kb + kBK <= kmax) {
 #pragma unroll
     for (int u = U0; u < U1; ++u) dma16(tile, d.off[u], dst + u * 1024);
   } else {
     const int nrow = kmax - kb;
+    const int lane = LEAN ? laundered_tid() & 63 : 0;
 #pragma unroll
-    for (int u = U0; u < U1; ++u)
-      dma16(tile, d.row[u] < nrow ? d.off[u] : static_cast<uint32_t>(d.col[u] * 2), dst + u * 1024);
+    for (int u = U0; u < U1; ++u) {
+      int row = d.row[u], col = d.col[u];
+      if constexpr (LEAN) stage_piece<D>(w, lane, u, row, col);
+      dma16(tile, row < nrow ? d.off[u] : static_cast<uint32_t>(col * 2), dst + u * 1024);
+    }
   }
 }
 
@@ -538,16 +559,6 @@ __device__ __forceinline__ bool merge_key_halves(const PrefillParams& p, char* s
   return true;
 }
 
-// The thread index passes through an empty asm so that everything derived
-// from it (operand addresses, staging offsets) is formed where it is used:
-// hoisted out of the persistent kernel's item loop, those values would stay
-// live across items and push the register count past 256.
-__device__ __forceinline__ int laundered_tid() {
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
-  return tid;
-}
-
 // Q^T operand of item `it` for this lane: row r = 32w + n, head dims
 // 16 ks + 8h .. +7 for MFMA step ks (zeros for padding rows).
 template <int D>
@@ -572,7 +583,7 @@ __device__ __forceinline__ void item_fetch_q(const PrefillParams& p, const ItemD
 
 // Per-wave staging constants of item `it`'s K/V tiles (waves 0..3 copy K,
 // 4..7 copy V).
-template <int KV, int D>
+template <int KV, int D, bool LEAN>
 struct ItemStaging {
   static constexpr bool PAGED = KV != kKvPacked;
   static constexpr bool FP8 = KV == kKvFp8;
@@ -605,12 +616,12 @@ struct ItemStaging {
     return tile_base<PAGED>(p, dbase, dstride, page, it.k_start, t * kBK);
   }
   __device__ __forceinline__ void copy(const PrefillParams& p, const ItemDesc& it, char* st, int page, int t) const {
-    dma_tile<Geom<D>::P>(st, tile(p, it, page, t), dl, t * kBK, it.kmax, w, v_skip);
+    dma_tile<D, LEAN>(st, tile(p, it, page, t), dl, t * kBK, it.kmax, w, v_skip);
   }
   // pieces [U0, U1) of this wave's share of tile t, whose first key is at src
   template <int U0, int U1>
   __device__ __forceinline__ void copy_part(const ItemDesc& it, char* st, const char* src, int t) const {
-    dma_tile<Geom<D>::P, U0, U1>(st, src, dl, t * kBK, it.kmax, w, v_skip);
+    dma_tile<D, LEAN, U0, U1>(st, src, dl, t * kBK, it.kmax, w, v_skip);
   }
   // fp8: load this lane's part of tile t (keys at or past kmax: the tile's first key, as
   // dma_tile), and write it to the tile's stage
@@ -635,10 +646,10 @@ struct ItemStaging {
 
 // Start the copies of item `it`'s tiles 0 and 1 into ring stages 0 and 1 (fp8: the loads
 // into raw; the prologue writes them).
-template <int KV, int D>
+template <int KV, int D, bool LEAN>
 __device__ __forceinline__ void item_fetch_tiles(const PrefillParams& p, char* smem_all, const ItemDesc& it,
                                                  Raw8 (&raw)[2]) {
-  const ItemStaging<KV, D> st(p, it);
+  const ItemStaging<KV, D, LEAN> st(p, it);
   constexpr bool PAGED = KV != kKvPacked;
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -758,8 +769,9 @@ __device__ __forceinline__ void store_rows_ahead(const PrefillParams& p, const I
 // item's rows go from the ring to the caches after the loop; `slot` is this thread's
 // row's slot, fetched before like the Q operands.
 // KV == kKvFp8: raw[0] and raw[1] are
-// the bytes of tiles 0 and 1, loaded before like the Q operands.
-template <int KV, int D, bool SPLIT, bool STORE>
+// the bytes of tiles 0 and 1, loaded before like the Q operands.  LEAN: fewer registers kept
+// (StageLane).
+template <int KV, int D, bool SPLIT, bool STORE, bool LEAN>
 __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_all, const ItemDesc& item,
                                             bf16x8 (&qop)[D / 16], const ItemDesc& next, uint32_t* claim_ctr,
                                             uint32_t& claim, int* s_slot, int& slot, Raw8 (&raw)[2]) {
@@ -830,7 +842,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
     vaddr[jd] = Gm::kVRing + (4 * h + (jl >> 2)) * RB +
                 ((2 * jd + ((lane >> 4) & 1)) ^ Gm::v_swz(jl >> 2)) * 32 + 8 * (jl & 3);
 
-  const ItemStaging<KV, D> stg(p, item);
+  const ItemStaging<KV, D, LEAN> stg(p, item);
   (void)s;
   (void)k_start;
   (void)kvh;
@@ -1061,7 +1073,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   if (next.valid) {
     item_fetch_q<D>(p, next, qop);
     if constexpr (STORE) slot = item_fetch_slot(p, next);
-    if constexpr (FP8) item_fetch_tiles<KV, D>(p, smem_all, next, raw);
+    if constexpr (FP8) item_fetch_tiles<KV, D, LEAN>(p, smem_all, next, raw);
   }
   if constexpr (STORE) {
     if (rows_in_ring(item)) item_store_rows<D>(p, item, smem_all, s_slot);
@@ -1074,7 +1086,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
   barrier_lds();  // every wave is done with the ring
   // stages 0 and 1 take the next item's first tiles
   if constexpr (!FP8) {
-    if (next.valid) item_fetch_tiles<KV, D>(p, smem_all, next, raw);
+    if (next.valid) item_fetch_tiles<KV, D, LEAN>(p, smem_all, next, raw);
   }
   // A work-queue grid claims the item after `next` here, one item ahead; the
   // caller reads the result after its own barrier, once the epilogue has run.
@@ -1114,8 +1126,17 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // on the same XCD (and its L2) whenever gridDim.x is a multiple of 8.  Tiles
 // past a sequence's end exit at once.  Used when the persistent grid's tables
 // would not fit its LDS.
-template <int KV, int D, bool STORE>
-__global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillParams p) {
+// PAIRED (D = 64): at most 128 registers, so that two workgroups fit a CU (the ring takes 64
+// KiB there): with more cells than CUs one's loads, barriers and softmax run under the
+// other's, where a single workgroup leaves them exposed; with fewer, the tighter
+// registers only cost (~10%: fewer operand reads in flight).  Heads 14/2, PAIRED against
+// not: 12 prompts of 100-1024 tokens (504 cells; Attention.forward) 24.0 -> 19.4 us; 32
+// prompts of 400 tokens after 1024 cached (768 cells, the persistent grid before) 82.6 ->
+// 70.8; one prompt of 2048 (114 cells) 28.4 -> 31.7; 24 prompts (1344 cells): 42 paired
+// against 35 on the persistent grid; one of 16000 (890 cells) 477 -> 485 (heads 16/16, 1008
+// cells: 544 -> 524).
+template <int KV, int D, bool STORE, bool PAIRED = false>
+__global__ __launch_bounds__(64 * kWaves, PAIRED ? 4 : 2) void varlen_prefill_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
   if constexpr (STORE) {
     if (blockIdx.x == 0 && blockIdx.y == 0) store_rows_outside<D>(p, p.cu_q[0], p.cu_q[p.num_seqs]);
@@ -1146,12 +1167,12 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_kernel(PrefillPara
   bf16x8 qop[D / 16];
   item_fetch_q<D>(p, it, qop);
   Raw8 raw[2] = {};
-  item_fetch_tiles<KV, D>(p, smem_all, it, raw);
+  item_fetch_tiles<KV, D, PAIRED>(p, smem_all, it, raw);
   if constexpr (STORE) slot = item_fetch_slot(p, it);
   ItemDesc none{};
   none.valid = false;
   uint32_t unused = 0;
-  prefill_run<KV, D, true, STORE>(p, smem_all, it, qop, none, nullptr, unused, s_slot, slot, raw);
+  prefill_run<KV, D, true, STORE, PAIRED>(p, smem_all, it, qop, none, nullptr, unused, s_slot, slot, raw);
 }
 
 // Persistent grid: one workgroup per CU walks the real work items.
@@ -1317,7 +1338,7 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
   int slot = -1;
   item_fetch_q<D>(p, cur, qop);
   Raw8 raw[2] = {};
-  item_fetch_tiles<KV, D>(p, smem_all, cur, raw);
+  item_fetch_tiles<KV, D, false>(p, smem_all, cur, raw);
   if constexpr (STORE) slot = item_fetch_slot(p, cur);
   for (int round = 1;; ++round) {
     // the next item is located (from the LDS tables) while this one's
@@ -1334,7 +1355,7 @@ __global__ __launch_bounds__(64 * kWaves) void varlen_prefill_persistent_kernel(
       nxt = desc_of(item64 < total ? static_cast<int>(item64) : total);
     }
     if constexpr (STORE) store_rows_ahead<D>(p, cur);
-    prefill_run<KV, D, false, STORE>(p, smem_all, cur, qop, nxt, claim_ctr, claim, s_slot, slot, raw);
+    prefill_run<KV, D, false, STORE, false>(p, smem_all, cur, qop, nxt, claim_ctr, claim, s_slot, slot, raw);
     if (!nxt.valid) break;
     cur = nxt;
   }
@@ -1378,8 +1399,11 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   // barriers) costs more than it saves (measured on config 2).
   const int64_t max_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
   const int cus = device_cu_count();
-  const bool persistent =
-      p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles && max_items > 2 * int64_t{cus};
+  // at D = 64 two workgroups fit a CU on the direct grid, worth it above one cell per CU
+  // and up to four (see PAIRED)
+  const bool paired = p.head_dim == 64 && max_items > cus && max_items <= 4 * int64_t{cus};
+  const bool persistent = p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles &&
+                          max_items > 2 * int64_t{cus} && !paired;
   // one workgroup per CU (the ring takes most of a CU's LDS); the work queue
   // needs whole XCD lanes
   const unsigned nw = static_cast<unsigned>(cus);
@@ -1444,17 +1468,21 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   const dim3 grid = p.split_tiles > 0
                         ? dim3(static_cast<unsigned>(max_items + pairs_split * p.num_kv_heads))
                         : dim3(static_cast<unsigned>(p.num_seqs * p.num_kv_heads), static_cast<unsigned>(p.num_q_tiles));
-#define NVA_DIRECT(PG, DD, ST) \
-  hipLaunchKernelGGL((varlen_prefill_kernel<PG, DD, ST>), grid, dim3(kThreads), 0, stream, p)
-  if (p.head_dim == 64) {
-    if (p.block_table) NVA_DIRECT(kKvPaged, 64, false);
-    else if (fuse) NVA_DIRECT(kKvPacked, 64, true);
-    else NVA_DIRECT(kKvPacked, 64, false);
+#define NVA_DIRECT(PG, DD, ST, PAIR) \
+  hipLaunchKernelGGL((varlen_prefill_kernel<PG, DD, ST, PAIR>), grid, dim3(kThreads), 0, stream, p)
+  if (p.head_dim == 64 && paired) {
+    if (p.block_table) NVA_DIRECT(kKvPaged, 64, false, true);
+    else if (fuse) NVA_DIRECT(kKvPacked, 64, true, true);
+    else NVA_DIRECT(kKvPacked, 64, false, true);
+  } else if (p.head_dim == 64) {
+    if (p.block_table) NVA_DIRECT(kKvPaged, 64, false, false);
+    else if (fuse) NVA_DIRECT(kKvPacked, 64, true, false);
+    else NVA_DIRECT(kKvPacked, 64, false, false);
   } else {
-    if (p.k_scale) NVA_DIRECT(kKvFp8, 128, false);
-    else if (p.block_table) NVA_DIRECT(kKvPaged, 128, false);
-    else if (fuse) NVA_DIRECT(kKvPacked, 128, true);
-    else NVA_DIRECT(kKvPacked, 128, false);
+    if (p.k_scale) NVA_DIRECT(kKvFp8, 128, false, false);
+    else if (p.block_table) NVA_DIRECT(kKvPaged, 128, false, false);
+    else if (fuse) NVA_DIRECT(kKvPacked, 128, true, false);
+    else NVA_DIRECT(kKvPacked, 128, false, false);
   }
 #undef NVA_DIRECT
   return hipGetLastError();

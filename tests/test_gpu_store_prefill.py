@@ -108,3 +108,27 @@ def test_keys_inside_the_cache_store_first(dev):
         outs.append((o, vc))
     assert torch.equal(outs[0][1], outs[1][1])
     assert float((outs[0][0].float() - outs[1][0].float()).abs().max()) < 2e-2
+
+
+@pytest.mark.parametrize("cells", ["one per CU", "above one", "four per CU", "above four"])
+@pytest.mark.parametrize("prefix", [0, 128])
+def test_head_dim_64_grids(dev, cells, prefix):
+    """Head dim 64 at the limits of its three grids (one workgroup per CU, two, the persistent
+    one): every output row against the oracle, packed and paged."""
+    from _helpers import assert_attn_close, f32, prefill_reference
+    from nanovllm_amd import workloads as W
+    import nanovllm_amd as nva
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    per_seq = 2 * 2  # 2 kv heads x 2 query tiles of 36 positions
+    seqs = {"one per CU": cus // per_seq, "above one": cus // per_seq + 1, "four per CU": 4 * cus // per_seq,
+            "above four": 4 * cus // per_seq + 1}[cells]
+    lens = [72 - (i % 3) * 35 for i in range(seqs)]
+    c = W.make_prefill_case(lens, 14, 2, 4 * seqs, prefix_len=prefix, block_size=64, head_dim=64, seed=seqs,
+                            bulk_device=dev, shared_prefix=False)
+    k, v = (c.k_cache, c.v_cache) if prefix else (c.k, c.v)
+    if prefix:
+        nva.store_kvcache(c.k, c.v, c.k_cache, c.v_cache, c.slot_mapping)
+    o = nva.flash_attn_varlen_func(c.q, k, v, c.max_seqlen_q, c.cu_seqlens_q, c.max_seqlen_k, c.cu_seqlens_k, c.scale,
+                                   block_table=c.block_tables)
+    torch.cuda.synchronize()
+    assert_attn_close(f32(o), prefill_reference(c), what=cells)
