@@ -798,10 +798,19 @@ __global__ __launch_bounds__(64) void paged_decode_spread_kernel(DecodeParams p)
 // monotonically).  Workgroup (0, 0) also stores the exclusive step prefix of
 // every sequence for the merge.  Grid: (P, head groups).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int shfl_up_i(int v, int d) {
-  const int lane = __lane_id();
-  const int src = lane >= d ? lane - d : lane;
-  return __builtin_amdgcn_ds_bpermute(src << 2, v);
+// Inclusive sum over the wavefront's lanes, by DPP row shifts and broadcasts (register to
+// register: a shuffle through the LDS crossbar costs ~100 cycles, and a scan is six of
+// them before the first load of a decode).  With the scans of a one-chunk batch done once and
+// 32-bit range divisions here and in the merge: 37 sequences of 256-4096 tokens, heads 32/8,
+// store included, 64.2 -> 61.4 us; 256 of 100-2048, heads 16/8, 190.2 -> 187.5.
+__device__ __forceinline__ int wave_scan_incl(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: rows of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15: rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31: rows 2, 3
+  return v;
 }
 
 // Inclusive scan over the workgroup (WAVES waves); `total` gets the sum.
@@ -809,11 +818,7 @@ template <int WAVES>
 __device__ __forceinline__ int block_scan_incl(int v, int* s_wsum, int& total) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = shfl_up_i(v, d);
-    if (lane >= d) v += t;
-  }
+  v = wave_scan_incl(v);
   if (lane == 63) s_wsum[wave] = v;
   __syncthreads();
   int before = 0;
@@ -828,7 +833,15 @@ __device__ __forceinline__ int block_scan_incl(int v, int* s_wsum, int& total) {
   return v + before;
 }
 
-__device__ __forceinline__ int64_t range_start(int64_t r, int64_t T, int64_t P) { return r * T / P; }
+// a * b / c for non-negative values, by a 32-bit division where the product allows it (a
+// 64-bit one is some 150 instructions, in front of the first loads).
+__device__ __forceinline__ int64_t mul_div(int64_t a, int64_t b, int64_t c) {
+  const uint64_t ab = static_cast<uint64_t>(a * b);
+  return ab >> 32 ? static_cast<int64_t>(ab / static_cast<uint64_t>(c))
+                  : static_cast<int64_t>(static_cast<uint32_t>(ab) / static_cast<uint32_t>(c));
+}
+
+__device__ __forceinline__ int64_t range_start(int64_t r, int64_t T, int64_t P) { return mul_div(r, T, P); }
 
 // Ranges used for T steps: the planned P, but no more than one per
 // kMinRangeSteps steps.  The host plans P from the block-table width, an upper
@@ -857,11 +870,12 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_balanced_kernel(Decod
 
   // pass 1: total step count T (and the prefix array for the merge)
   int T = 0;
+  int st = 0, incl = 0;  // of the last chunk: all of them when the batch fits one
   for (int c0 = 0; c0 < B; c0 += CH) {
     const int b = c0 + tid;
-    const int st = b < B ? (clamped_len(p, b) + 31) >> 5 : 0;
+    st = b < B ? (clamped_len(p, b) + 31) >> 5 : 0;
     int tot;
-    const int incl = block_scan_incl<WAVES>(st, s_wsum, tot);
+    incl = block_scan_incl<WAVES>(st, s_wsum, tot);
     if (write_prefix && b < B) p.ws_prefix[b] = T + incl - st;
     T += tot;
   }
@@ -876,9 +890,11 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_balanced_kernel(Decod
   int carry = 0;
   for (int c0 = 0; c0 < B && carry < end; c0 += CH) {
     const int b = c0 + tid;
-    const int st = b < B ? (clamped_len(p, b) + 31) >> 5 : 0;
-    int tot;
-    const int incl = block_scan_incl<WAVES>(st, s_wsum, tot);
+    int tot = T;
+    if (B > CH) {  // a batch of one chunk was scanned in pass 1
+      st = b < B ? (clamped_len(p, b) + 31) >> 5 : 0;
+      incl = block_scan_incl<WAVES>(st, s_wsum, tot);
+    }
     const int s0 = carry + incl - st;  // first step of sequence b
     const int s1 = carry + incl;
     const bool hit = b < B && st > 0 && s0 < end && s1 > start;
@@ -959,8 +975,13 @@ __global__ __launch_bounds__(64 * kMergeHeads) void decode_merge_kernel(DecodePa
       zero = true;
       first = count = 0;
     } else {
-      const int64_t rf = ((s0 + 1) * P - 1) / T;  // range holding step s0
-      const int64_t rl = (s1 * P - 1) / T;        // range holding step s1 - 1
+      // range holding step s0, and step s1 - 1 (mul_div with the product less one)
+      auto range_of = [&](int64_t end) {
+        const uint64_t x = static_cast<uint64_t>(end * P - 1);
+        return x >> 32 ? static_cast<int64_t>(x / static_cast<uint64_t>(T))
+                       : static_cast<int64_t>(static_cast<uint32_t>(x) / static_cast<uint32_t>(T));
+      };
+      const int64_t rf = range_of(s0 + 1), rl = range_of(s1);
       if (rf == rl) return;
       first = b + rf;
       count = rl - rf + 1;
@@ -973,14 +994,8 @@ __global__ __launch_bounds__(64 * kMergeHeads) void decode_merge_kernel(DecodePa
   }
   if (h >= p.num_heads) return;
   if (zero && p.new_k && h % p.group == 0 && (!WIDE || wq == 0)) store_empty_rows_wave(p, b, h / p.group, lane);
-  // A partial slot holds data unless it is a balanced range with no steps (P > T).
-  const int64_t T = p.balanced_ranges > 0 ? p.ws_prefix[p.batch] : 0;
-  const int64_t PU = p.balanced_ranges > 0 ? used_ranges(p.balanced_ranges, T) : 0;
-  auto has_data = [&](int64_t s) {
-    if (p.balanced_ranges <= 0) return true;
-    const int64_t rr = first - b + s;
-    return range_start(rr, T, PU) != range_start(rr + 1, T, PU);
-  };
+  // (Every slot of [first, first + count) holds a partial: used_ranges leaves no range
+  // without steps.)
   const bool cols = 2 * lane < p.head_dim;  // lane owns output columns 2 lane, 2 lane + 1
   float M = kNegInf, L = 0.f, o0 = 0.f, o1 = 0.f;
   const int64_t s_lo = WIDE ? count * wq / kMergeHeads : 0;
@@ -991,7 +1006,7 @@ __global__ __launch_bounds__(64 * kMergeHeads) void decode_merge_kernel(DecodePa
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int64_t s = s0 + u;
-        const bool ok = s < s_hi && has_data(s);
+        const bool ok = s < s_hi;
         const int64_t idx = (first + (ok ? s : 0)) * p.num_heads + h;
         ml[u] = ok ? *reinterpret_cast<const f32x2*>(p.ws_ml + idx * 2) : f32x2{kNegInf, 0.f};
         v[u] = ok && cols ? *reinterpret_cast<const f32x2*>(p.ws_o + idx * p.head_dim + 2 * lane) : f32x2{0.f, 0.f};
