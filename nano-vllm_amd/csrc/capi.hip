@@ -471,6 +471,7 @@ int decode_impl(const void* q, int64_t q_row_stride, const void* k_cache, const 
   p.num_splits = plan.num_splits;
   p.balanced_ranges = plan.balanced_ranges;
   p.spread = plan.spread;
+  p.spread_short = plan.spread_short;
   p.head_dim = head_dim;
   p.scale_log2 = softmax_scale * kLog2e;
   p.kv_fp8 = kv_dtype == NVA_DTYPE_FP8_E4M3 ? 1 : 0;

@@ -50,6 +50,7 @@ struct DecodeParams {
   int32_t num_splits;         // fixed mode: splits per sequence
   int32_t balanced_ranges;    // balanced mode: number of step ranges P (0 = fixed mode)
   int32_t spread;             // > 0: spread mode with that many shares per sequence (small batches)
+  int32_t spread_short;       // spread mode over a table of `spread` steps: one workgroup per (sequence, kv head)
   int32_t head_dim;           // 64 or 128
   // Store fused into the decode launch (null new_k: none): row b of new_k /
   // new_v (bf16, nkv * d elements) goes to cache slot slot_mapping[b].  Rows
@@ -229,6 +230,7 @@ struct DecodePlan {
   int32_t num_splits;
   int32_t balanced_ranges;
   int32_t spread;             // > 0: spread mode, shares per sequence
+  int32_t spread_short;       // spread mode, and the table has no more steps than shares (at most kShortSteps)
   int64_t partial_slots;      // partial (O, max, sum) slots the workspace holds
 };
 // Spread mode (small batches): the largest batch * num_kv_heads it serves, the
@@ -240,6 +242,7 @@ constexpr int kSpreadTargetWaves = 1024;
 // (captured batch 1, context 1024: 16 shares 9.6 us per layer, 8 shares 10.6, 32 shares 11.6).
 constexpr int kSpreadMaxShares = 16;
 constexpr int kWgMaxBlocks = 64;
+constexpr int kShortSteps = 8;  // waves of a short-table workgroup
 
 DecodePlan plan_decode(int32_t batch, int32_t num_kv_heads, int32_t max_blocks,
                        int32_t block_size, int32_t kv_dtype, int32_t requested_splits);

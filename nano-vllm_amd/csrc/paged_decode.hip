@@ -786,6 +786,173 @@ __global__ __launch_bounds__(64) void paged_decode_spread_kernel(DecodeParams p)
   if (g == 0) *reinterpret_cast<f32x2*>(p.ws_ml + idx * 2) = f32x2{m_run, l};
 }
 
+// The new token's K and V rows of (b, kvh) for a sequence with no keys, when
+// the store is fused into the decode launch: no decode wave reads key ctx-1 of
+// such a sequence, so the merge kernel -- stream-ordered after every read of
+// the decode launch -- stores them.  One wave: lanes 0..d/8-1 write the key
+// row, lanes 32..32+d/8-1 the value row, 8 elements each (fp8: quantised as
+// the store kernel does).  Slots outside the pool are skipped.
+__device__ void store_empty_rows_wave(const DecodeParams& p, int b, int kvh, int lane) {
+  const int64_t slot = p.slot_mapping[b];
+  const int j = lane & 31;
+  if (slot < 0 || slot >= p.num_blocks * p.block_size || 8 * j >= p.head_dim) return;
+  const bool is_v = lane >= 32;
+  const u32x4 x = ld16((is_v ? p.new_v + b * p.new_v_stride : p.new_k + b * p.new_k_stride) +
+                       static_cast<int64_t>(kvh) * p.head_dim + 8 * j);
+  const int64_t elem = (slot * p.num_kv_heads + kvh) * p.head_dim + 8 * j;
+  char* base = static_cast<char*>(const_cast<void*>(is_v ? p.v_cache : p.k_cache));
+  if (p.kv_fp8)
+    *reinterpret_cast<u32x2*>(base + elem) = bf16x8_to_e4m3fn(x, is_v ? p.v_scale[kvh] : p.k_scale[kvh]);
+  else
+    *reinterpret_cast<u32x4*>(base + 2 * elem) = x;
+}
+
+// ---------------------------------------------------------------------------
+// Short tables (spread_short: at most kShortSteps steps per sequence, a share each):
+// one workgroup per (sequence, kv head), a wave per step, merged through LDS instead
+// of a second launch.  The arithmetic is that of the spread kernel and its merge, in the
+// same order, so the results are bit-identical.  One CU moves a pair's steps (at most
+// 128 KiB) slower than eight do, by 2-3 us at eight steps; the merge launch that this
+// saves costs more.  Attention.forward, captured / eager, heads 16/8: 1 sequence of 30 tokens
+// 6.2 -> 3.7 / 10.0 -> 6.9 us, of 256 7.5 -> 6.2 / 10.0 -> 6.9, 16 of 256 10.8 -> 8.9 / 11.6 ->
+// 9.1; heads 64/8 over fp8, 16 of 256, 11.8 -> 8.4 / 12.1 -> 8.6.
+// With a store it needs store_exact: an empty sequence's row is then written here,
+// since whoever reads its slot writes it first.  Grid: (num_kv_heads, batch).
+// ---------------------------------------------------------------------------
+template <bool FP8, int D, bool STORE>
+__global__ __launch_bounds__(64 * kShortSteps) void paged_decode_short_kernel(DecodeParams p) {
+  constexpr int EB = FP8 ? 1 : 2;
+  constexpr int kHeads = 16;  // query heads of a kv head, at most
+  __shared__ __attribute__((aligned(16))) float s_o[kShortSteps][kHeads][D + 4];  // rows 4 banks apart
+  __shared__ float s_m[kShortSteps][kHeads], s_l[kShortSteps][kHeads];
+  const int kvh = blockIdx.x;
+  const int b = blockIdx.y;
+  const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 15;
+  const int g = lane >> 4;
+  const int bt_row = lane < p.max_blocks ? p.block_table[b * p.bt_row_stride + lane] : -1;
+  const int ctx = __builtin_amdgcn_readfirstlane(clamped_len(p, b));
+  const int shares = (ctx + 31) >> 5;
+  const float vscale = FP8 ? p.v_scale[kvh] : 1.0f;
+  const int h = kvh * p.group + n;
+  const bool cols = n < p.group && 32 * g < D;  // lanes holding a head's output columns
+  if (r < shares) {
+    const int k_begin = 32 * r;
+    const int k_end = min(ctx, k_begin + 32);
+    bool stores = false;
+    NewRow<FP8, D> nr;
+    u32x4 x = {0u, 0u, 0u, 0u};
+    if constexpr (STORE) {
+      const int64_t slot = __builtin_amdgcn_readfirstlane(p.slot_mapping[b]);
+      store_rows_read_here<FP8, D>(p, kvh, b, ctx, k_begin, k_end, bt_row);
+      stores = r == shares - 1 && slot >= 0 && slot < static_cast<int64_t>(p.num_blocks) * p.block_size;
+      if (stores) {
+        const uint16_t* kin = p.new_k + b * p.new_k_stride + kvh * D;
+        const uint16_t* vin = p.new_v + b * p.new_v_stride + kvh * D;
+        nr.load(kin, vin, n, g, FP8 ? p.k_scale[kvh] : 1.f, FP8 ? p.v_scale[kvh] : 1.f);
+        x = ld16((lane >= 32 ? vin : kin) + 8 * (lane & (D / 8 - 1)));
+        nr.step = 0;
+        nr.row = (ctx - 1) & 31;
+        nr.slot = static_cast<int>(slot);
+      }
+    }
+    WaveItem w;
+    w.slot_bytes = static_cast<int64_t>(p.num_kv_heads) * D * EB;
+    w.kbase = static_cast<const char*>(p.k_cache) + static_cast<int64_t>(kvh) * D * EB;
+    w.vbase = static_cast<const char*>(p.v_cache) + static_cast<int64_t>(kvh) * D * EB;
+    w.bt = nullptr;
+    w.num_blocks = p.num_blocks;
+    w.block_size = p.block_size;
+    w.k_begin = k_begin;
+    w.k_end = k_end;
+    w.krow0 = 8 * (n >> 2) + (n & 3);
+    w.n = n;
+    w.g = g;
+    StepRegs<FP8> A;
+    const StepRsrc rs = step_rsrc<true, D * EB>(w, 0, 1, bt_row);
+    load_step_buf<FP8, D>(A, w, rs);
+    bf16x8 qop[4];
+    const uint16_t* qrow = p.q + b * p.q_row_stride + h * D;
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+      const u32x4 z = {0u, 0u, 0u, 0u};
+      qop[s] = as_bf16x8(n < p.group ? ld16(qrow + qk_dim<FP8>(s, g)) : z);
+    }
+    const float sl2 = FP8 ? p.scale_log2 * p.k_scale[kvh] : p.scale_log2;
+    f32x4 acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = kNegInf, l = 0.f;
+    if (STORE && stores) nr.apply(A, 0, rs.row0);
+    compute_step<FP8, D, false>(A, rs.nvalid, g, qop, sl2, acc, m_run, l);
+    l += shfl_xor(l, 16);
+    l += shfl_xor(l, 32);
+    if constexpr (STORE) {
+      if (stores) store_row_wave<FP8, D>(p, kvh, nr.slot, x);
+    }
+    if (shares == 1) {
+      if (!cols) return;
+      const float inv = l > 0.f ? vscale / l : 0.f;
+      uint16_t* orow = p.out + b * p.out_row_stride + h * D + 32 * g;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        u32x4 o;
+#pragma unroll
+        for (int q2 = 0; q2 < 4; ++q2) o[q2] = pack_bf16x2(acc[2 * q2][q] * inv, acc[2 * q2 + 1][q] * inv);
+        st16(orow + 8 * q, o);
+      }
+      return;
+    }
+    if (cols) {
+      float* wo = &s_o[r][n][32 * g];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 lo, hi;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          lo[j] = acc[j][q] * vscale;
+          hi[j] = acc[4 + j][q] * vscale;
+        }
+        *reinterpret_cast<f32x4*>(wo + 8 * q) = lo;
+        *reinterpret_cast<f32x4*>(wo + 8 * q + 4) = hi;
+      }
+      if (g == 0) {
+        s_m[r][n] = m_run;
+        s_l[r][n] = l;
+      }
+    }
+  } else if (shares == 0) {  // no keys: zeros, and the new row
+    if (r != 0) return;
+    if (STORE) store_empty_rows_wave(p, b, kvh, lane);
+    if (!cols) return;
+    uint16_t* orow = p.out + b * p.out_row_stride + h * D + 32 * g;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) st16(orow + 8 * q, u32x4{0u, 0u, 0u, 0u});
+    return;
+  }
+  if (shares <= 1) return;  // uniform over the workgroup
+  __syncthreads();
+  // two output columns per lane, one head at a time per wave
+  for (int hd = r; hd < p.group; hd += static_cast<int>(blockDim.x >> 6)) {
+    if (2 * lane >= D) break;
+    float M = kNegInf;
+    for (int u = 0; u < shares; ++u) M = fmaxf(M, s_m[u][hd]);
+    float L = 0.f, o0 = 0.f, o1 = 0.f;
+    if (M != kNegInf) {  // otherwise no valid key
+      for (int u = 0; u < shares; ++u) {
+        const float wt = fast_exp2(s_m[u][hd] - M);
+        L += wt * s_l[u][hd];
+        o0 += wt * s_o[u][hd][2 * lane];
+        o1 += wt * s_o[u][hd][2 * lane + 1];
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    *reinterpret_cast<uint32_t*>(p.out + b * p.out_row_stride + (kvh * p.group + hd) * D + 2 * lane) =
+        pack_bf16x2(o0 * inv, o1 * inv);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Balanced split-K.  Every sequence is cut into 32-key steps and the steps of
 // all sequences, in sequence order, form one list of T entries (T from a
@@ -937,27 +1104,6 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_balanced_kernel(Decod
 // sequence: 16.7 us as one wave per head).
 constexpr int kMergeHeads = 4;    // heads (waves) per merge workgroup
 constexpr int kMergeWideMin = 8;  // ranges per sequence (on average) from which the merge is WIDE
-
-// The new token's K and V rows of (b, kvh) for a sequence with no keys, when
-// the store is fused into the decode launch: no decode wave reads key ctx-1 of
-// such a sequence, so the merge kernel -- stream-ordered after every read of
-// the decode launch -- stores them.  One wave: lanes 0..d/8-1 write the key
-// row, lanes 32..32+d/8-1 the value row, 8 elements each (fp8: quantised as
-// the store kernel does).  Slots outside the pool are skipped.
-__device__ void store_empty_rows_wave(const DecodeParams& p, int b, int kvh, int lane) {
-  const int64_t slot = p.slot_mapping[b];
-  const int j = lane & 31;
-  if (slot < 0 || slot >= p.num_blocks * p.block_size || 8 * j >= p.head_dim) return;
-  const bool is_v = lane >= 32;
-  const u32x4 x = ld16((is_v ? p.new_v + b * p.new_v_stride : p.new_k + b * p.new_k_stride) +
-                       static_cast<int64_t>(kvh) * p.head_dim + 8 * j);
-  const int64_t elem = (slot * p.num_kv_heads + kvh) * p.head_dim + 8 * j;
-  char* base = static_cast<char*>(const_cast<void*>(is_v ? p.v_cache : p.k_cache));
-  if (p.kv_fp8)
-    *reinterpret_cast<u32x2*>(base + elem) = bf16x8_to_e4m3fn(x, is_v ? p.v_scale[kvh] : p.k_scale[kvh]);
-  else
-    *reinterpret_cast<u32x4*>(base + 2 * elem) = x;
-}
 
 template <bool WIDE>
 __global__ __launch_bounds__(64 * kMergeHeads) void decode_merge_kernel(DecodeParams p) {
@@ -1148,6 +1294,7 @@ DecodePlan plan_decode(int32_t batch, int32_t num_kv_heads, int32_t max_blocks, 
     plan.num_splits = 1;
     plan.balanced_ranges = 0;
     plan.spread = static_cast<int32_t>(S);
+    plan.spread_short = S > 1 && S == table_steps && S <= kShortSteps;
     plan.partial_slots = S > 1 ? static_cast<int64_t>(batch) * S : 0;
     return plan;
   }
@@ -1195,6 +1342,15 @@ static hipError_t launch_decode_t(const DecodeParams& p, hipStream_t stream) {
   else                                                                                                  \
     hipLaunchKernelGGL((KERNEL<FP8, 1, PF, D EXTRA>), GRID, dim3(64), 0, stream, p);
   bool merge;
+  if (p.spread_short && (!p.new_k || p.store_exact)) {
+    const dim3 grid(static_cast<unsigned>(p.num_kv_heads), static_cast<unsigned>(p.batch));
+    const dim3 block(static_cast<unsigned>(64 * p.spread));
+    if (p.new_k)
+      hipLaunchKernelGGL((paged_decode_short_kernel<FP8, D, true>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((paged_decode_short_kernel<FP8, D, false>), grid, block, 0, stream, p);
+    return hipGetLastError();
+  }
   if (p.spread > 0) {
     const dim3 grid(static_cast<unsigned>(p.spread), static_cast<unsigned>(p.num_kv_heads),
                     static_cast<unsigned>(p.batch));

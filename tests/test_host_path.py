@@ -157,6 +157,51 @@ def test_decode_equals_store_then_decode(dev, monkeypatch, slots, B, nh, nkv, d,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,nh,nkv,d,fp8,bs,width", [
+    (1, 16, 8, 128, False, 256, 1), (10, 16, 8, 128, False, 256, 1), (16, 64, 8, 128, True, 128, 2),
+    (10, 128, 8, 128, False, 32, 8), (60, 14, 2, 64, False, 256, 1), (128, 4, 1, 128, True, 32, 5),
+    (9, 16, 8, 128, False, 32, 2), (20, 5, 5, 64, False, 64, 3)])
+@pytest.mark.parametrize("slots", ["own", "rolled", "empty rows"])
+def test_short_tables_in_one_launch(dev, B, nh, nkv, d, fp8, bs, width, slots):
+    """Tables of at most eight steps: one workgroup per (sequence, kv head), bit-identical to the
+    spread kernel and its merge (store_and_decode keeps those), with and without the store,
+    and equal to the oracle."""
+    import nanovllm_amd as nva
+    from _helpers import FP8_MAX_ABS, assert_attn_close, decode_reference, f32
+    from nanovllm_amd import workloads as W
+    cap = bs * width
+    base = [1, 31, 0, 32, 33, cap, cap - 1, cap // 2, 2, min(cap, 64)]
+    lens = [base[i % len(base)] for i in range(B)]
+    c = W.make_decode_case(B, nh, nkv, 0, 0, B * width + 2, head_dim=d, fp8=fp8, seed=B + d, bulk_device=dev,
+                           block_size=bs, lengths=lens, table_width=width)
+    live = [b for b, n in enumerate(lens) if n > 0]
+    s = c.slot_mapping
+    if slots == "rolled":
+        s[live] = s[live].roll(1)
+    elif slots == "empty rows":  # to slots past the live keys: nobody reads them
+        used = set(c.block_tables.flatten().tolist())
+        free = [i for i in range(B * width + 2) if i not in used]
+        for i, b in enumerate(b for b, n in enumerate(lens) if n == 0):
+            s[b] = free[i // bs] * bs + i % bs
+    tol = dict(max_abs=FP8_MAX_ABS, mean_abs=FP8_MAX_ABS) if fp8 else {}
+    args = dict(softmax_scale=c.scale, k_scale=c.k_scale, v_scale=c.v_scale)
+    layer = _layer(c, c.k_cache.clone(), c.v_cache.clone(), (c.k_scale, c.v_scale))
+    nva.set_context(False, slot_mapping=s, context_lens=c.context_lens, block_tables=c.block_tables)
+    one = layer(c.q, c.k_new, c.v_new).view(B, nh, d)
+    nva.reset_context()
+    if slots != "rolled":
+        kc, vc = c.k_cache.clone(), c.v_cache.clone()
+        spread = nva.store_and_decode(c.q.unsqueeze(1), c.k_new, c.v_new, kc, vc, s, c.context_lens, c.block_tables, **args)
+        torch.cuda.synchronize()
+        _same((spread[:, 0], kc, vc), (one, layer.k_cache, layer.v_cache))
+    nva.store_kvcache(c.k_new, c.v_new, c.k_cache, c.v_cache, s, c.k_scale, c.v_scale)
+    two = nva.flash_attn_with_kvcache(c.q.unsqueeze(1), c.k_cache, c.v_cache, c.context_lens, c.block_tables, **args)
+    torch.cuda.synchronize()
+    _same((two[:, 0], c.k_cache, c.v_cache), (one, layer.k_cache, layer.v_cache))
+    assert_attn_close(f32(one), decode_reference(c), what=f"short {B} {nh}/{nkv} d={d}", **tol)
+
+
+@pytest.mark.gpu
 def test_producer_equals_the_general_path(dev, monkeypatch):
     from nanovllm_amd import workloads as W
     from nanovllm_amd.layers.qk_norm_rope import qk_norm_rope
