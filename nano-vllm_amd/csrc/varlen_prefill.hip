@@ -1393,12 +1393,32 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   const bool nothing = p0.num_seqs <= 0 || max_seqlen_q <= 0;
   PrefillParams p = p0;
   p.positions_per_tile = prefill_positions_per_tile(p.group);
-  p.num_q_tiles = nothing ? 0 : (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile;
+  const int cus = device_cu_count();
+  auto q_tiles = [&]() { return nothing ? 0 : (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile; };
+  p.num_q_tiles = q_tiles();
+  // max_seqlen_k only sizes the cuts: a wrong value changes which items are
+  // halved or split, never the result beyond rounding
+  const int64_t kt_max = (std::max<int64_t>(max_seqlen_k, 0) + kBK - 1) / kBK;
+  // Half the rows per item for a launch that leaves CUs idle: with 128 rows each SIMD runs
+  // one wave, and a key tile takes ~1.25 us instead of ~1.8, as do the item's first loads,
+  // merge and stores.  Where key halves want the idle CUs too, only up to 3/8 of the CUs
+  // (1/8 at d = 64, whose shorter tiles gain less).  Full -> half rows, d = 128: one prompt
+  // of 128 tokens, heads 16/8, 10.1 -> 8.2 us (8 items), 4 of 300 14.2 -> 12.4 (96), one of
+  // 1024 26.0 -> 22.9 (64), heads 4/1, 25.0 -> 21.5; 500 after 4096 cached 65 -> 50 (32); at
+  // 128 items one of 2048, heads 16/8, 37.5 -> 35.9, of 1024, 32/8, 27.5 -> 28.9, and of 500,
+  // 64/8, 20.6 -> 26.3.  d = 64, heads 14/2: 4 of 300 9.9 -> 8.2 (72, too short for key
+  // halves), one of 500 13.8 -> 13.0 (28), of 1024 18.9 -> 19.4 (58), of 2048 28.2 -> 48.8
+  // (114).
+  const int64_t full_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
+  const int eighths = kt_max < kSplitMin ? 4 : (p.head_dim == 64 ? 1 : 3);
+  if (8 * full_items <= eighths * int64_t{cus} && p.positions_per_tile > 1) {
+    p.positions_per_tile /= 2;
+    p.num_q_tiles = q_tiles();
+  }
   // Persistent grid when there are enough items to balance; with at most two
   // per CU its table set-up (one more dependent global load and a few
   // barriers) costs more than it saves (measured on config 2).
   const int64_t max_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
-  const int cus = device_cu_count();
   // at D = 64 two workgroups fit a CU on the direct grid, worth it above one cell per CU
   // and up to four (see PAIRED)
   const bool paired = p.head_dim == 64 && max_items > cus && max_items <= 4 * int64_t{cus};
@@ -1449,9 +1469,6 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
 #undef NVA_PERSIST
     return hipGetLastError();
   }
-  // max_seqlen_k only sizes the cut: a wrong value changes which items are
-  // split, never the result beyond rounding
-  const int64_t kt_max = (std::max<int64_t>(max_seqlen_k, 0) + kBK - 1) / kBK;
   p.split_tiles = 0;
   p.split_slots = kPrefillSplitSlots;
   p.split_cus = cus;

@@ -132,3 +132,35 @@ def test_head_dim_64_grids(dev, cells, prefix):
                                    block_table=c.block_tables)
     torch.cuda.synchronize()
     assert_attn_close(f32(o), prefill_reference(c), what=cells)
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(16, 8, 128), (32, 8, 128), (24, 8, 128), (7, 1, 128), (8, 8, 128), (14, 2, 64)])
+@pytest.mark.parametrize("prefix", [0, 512])
+@pytest.mark.parametrize("over", [0, 1], ids=["half rows", "full rows"])
+def test_half_row_items(dev, nh, nkv, d, prefix, over):
+    """Small launches run items of half the rows: the last size that does and the first that does
+    not, with keys enough for key halves (a long first sequence), every row against the oracle."""
+    from _helpers import assert_attn_close, f32, prefill_reference
+    from nanovllm_amd import workloads as W
+    import nanovllm_amd as nva
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    bp = 256 // (nh // nkv)
+    items = (3 if d == 128 else 1) * cus // 8  # of full rows, at most
+    tiles = 2 if prefix or bp >= 256 else -(-512 // bp)  # of the longest sequence
+    seqs = max(1, items // (nkv * tiles)) + over
+    if not over and seqs * nkv * tiles * 8 > (3 if d == 128 else 1) * cus:
+        pytest.skip("one sequence is above the limit")
+    lens = [tiles * bp - 3] + [max(1, (37 * i) % (tiles * bp)) for i in range(1, seqs)]
+    c = W.make_prefill_case(lens, nh, nkv, sum(-(-(n + prefix) // 128) for n in lens) + 2, prefix_len=prefix, block_size=128,
+                            head_dim=d, seed=seqs, bulk_device=dev, shared_prefix=False)
+    layer = nva.Attention(nh, d, c.scale, nkv)
+    layer.k_cache, layer.v_cache = c.k_cache, c.v_cache
+    for _ in range(2):
+        nva.set_context(True, c.cu_seqlens_q, c.cu_seqlens_k, c.max_seqlen_q, c.max_seqlen_k, c.slot_mapping, None,
+                        c.block_tables)
+        o = layer(c.q, c.k, c.v).view(-1, nh, d)
+        nva.reset_context()
+        torch.cuda.synchronize()
+        assert_attn_close(f32(o), prefill_reference(c), what=f"{seqs} sequences")
+    rows = c.k_cache.view(-1, nkv, d)[c.slot_mapping.long()]
+    assert torch.equal(rows, c.k)
