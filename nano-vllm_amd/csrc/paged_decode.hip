@@ -969,7 +969,10 @@ __global__ __launch_bounds__(64 * kShortSteps) void paged_decode_short_kernel(De
 // register: a shuffle through the LDS crossbar costs ~100 cycles, and a scan is six of
 // them before the first load of a decode).  With the scans of a one-chunk batch done once and
 // 32-bit range divisions here and in the merge: 37 sequences of 256-4096 tokens, heads 32/8,
-// store included, 64.2 -> 61.4 us; 256 of 100-2048, heads 16/8, 190.2 -> 187.5.
+// store included, 64.2 -> 61.4 us; 256 of 100-2048, heads 16/8, 190.2 -> 187.5.  The kernel
+// with the store inside scans again in its second pass: lengths kept across the passes cost it
+// more in registers than the scan (256 captured sequences of 1024 tokens, heads 16/8, a
+// layer: 184.8 us kept, 180.4 scanned again; 64 of them 53.5 and 52.5).
 __device__ __forceinline__ int wave_scan_incl(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: rows of 16 lanes
   v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
@@ -1058,7 +1061,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_decode_balanced_kernel(Decod
   for (int c0 = 0; c0 < B && carry < end; c0 += CH) {
     const int b = c0 + tid;
     int tot = T;
-    if (B > CH) {  // a batch of one chunk was scanned in pass 1
+    if (STORE || B > CH) {  // plain: a batch of one chunk was scanned in pass 1
       st = b < B ? (clamped_len(p, b) + 31) >> 5 : 0;
       incl = block_scan_incl<WAVES>(st, s_wsum, tot);
     }
