@@ -1129,12 +1129,19 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // PAIRED (D = 64): at most 128 registers, so that two workgroups fit a CU (the ring takes 64
 // KiB there): with more cells than CUs one's loads, barriers and softmax run under the
 // other's, where a single workgroup leaves them exposed; with fewer, the tighter
-// registers only cost (~10%: fewer operand reads in flight).  Heads 14/2, PAIRED against
-// not: 12 prompts of 100-1024 tokens (504 cells; Attention.forward) 24.0 -> 19.4 us; 32
-// prompts of 400 tokens after 1024 cached (768 cells, the persistent grid before) 82.6 ->
-// 70.8; one prompt of 2048 (114 cells) 28.4 -> 31.7; 24 prompts (1344 cells): 42 paired
-// against 35 on the persistent grid; one of 16000 (890 cells) 477 -> 485 (heads 16/16, 1008
-// cells: 544 -> 524).
+// registers only cost (~10%: fewer operand reads in flight).  Up to two cells per CU the
+// alternative is this grid unpaired, where an item has a CU to itself and the lightest wait
+// for one; above two, the persistent grid, which evens out items of unequal work: two
+// heavy items on one CU set the length of a paired launch.  Attention.forward, heads 14/2, unpaired
+// (above 512 cells persistent) -> PAIRED, us.
+//   256 to 512 cells: 12 prompts of 100-1024 tokens 23.2 -> 18.9, 10 of 500 21.9 -> 17.8, 8 of
+//   128-1024 25.8 -> 21.6, 40 of 200 after 256 cached 28.6 -> 27.0; 12 of 350-700 21.4 -> 23.6;
+//   even items above 12 tiles, 5 of 1024 22.4 -> 26.7, 8 of 1024 28.9 -> 30.1; above 16 tiles,
+//   6 of 700-1400 27.0 -> 34.7, 4 of 2000 40.7 -> 47.6, one of 8000 127 -> 163.
+//   Up to 1024 cells: 24 of 300-700 36.0 -> 28.2, 32 of 400 after 1024 cached 87.5 -> 75.8; even,
+//   8 of 2000 86.4 -> 73.0, one of 10000 252 -> 222; above 28 tiles and not even, 4 of 500-4600
+//   100 -> 128, 8 of 600-2200 65.6 -> 70.4, 16 of 100-700 after 2048 cached 97 -> 112.
+//   1344 cells, 24 prompts: 35 -> 42.
 template <int KV, int D, bool STORE, bool PAIRED = false>
 __global__ __launch_bounds__(64 * kWaves, PAIRED ? 4 : 2) void varlen_prefill_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(1024))) char smem_all[kStages * Geom<D>::kStageBytes];
@@ -1387,6 +1394,11 @@ constexpr int kSplitNum = 3;
 constexpr int kSplitDen = 5;
 constexpr int kSplitMin = 8;
 constexpr int kSplitMaxPageTiles = 8;  // paged key halving for block sizes up to 512
+// Longest context, in key tiles, of a PAIRED launch: up to two cells per CU, the same with
+// items known to be even, and above two.
+constexpr int kPairedTiles = 16;
+constexpr int kPairedTilesEven = 12;
+constexpr int kPairedTilesTwo = 28;
 
 hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seqlen_k, hipStream_t stream,
                           const StoreParams* store, int store_vec) {
@@ -1419,9 +1431,17 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   // per CU its table set-up (one more dependent global load and a few
   // barriers) costs more than it saves (measured on config 2).
   const int64_t max_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
-  // at D = 64 two workgroups fit a CU on the direct grid, worth it above one cell per CU
-  // and up to four (see PAIRED)
-  const bool paired = p.head_dim == 64 && max_items > cus && max_items <= 4 * int64_t{cus};
+  // At D = 64 two workgroups fit a CU on the direct grid (see PAIRED, also for the figures
+  // that place these limits): above one cell per CU while the contexts are short, and above
+  // two, up to four, at any length where the items' work is known to be even -- one sequence,
+  // or fresh rows (the store's, the only count of them here) that fill 4/5 of num_seqs *
+  // max_seqlen_q.
+  const bool even = p.num_seqs == 1 || (store != nullptr && !p.block_table &&
+                                        5 * store->num_tokens >= 4 * int64_t{p.num_seqs} * max_seqlen_q);
+  const bool paired =
+      p.head_dim == 64 && max_items > cus &&
+      (max_items <= 2 * int64_t{cus} ? kt_max <= (even ? kPairedTilesEven : kPairedTiles)
+                                     : max_items <= 4 * int64_t{cus} && (even || kt_max <= kPairedTilesTwo));
   const bool persistent = p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles &&
                           max_items > 2 * int64_t{cus} && !paired;
   // one workgroup per CU (the ring takes most of a CU's LDS); the work queue
