@@ -1394,6 +1394,9 @@ constexpr int kSplitNum = 3;
 constexpr int kSplitDen = 5;
 constexpr int kSplitMin = 8;
 constexpr int kSplitMaxPageTiles = 8;  // paged key halving for block sizes up to 512
+// Half-row items (launch_prefill): contexts above so many key tiles are cut in halves.
+constexpr int kHalfRowsSplit = 16;
+constexpr int kHalfRowsSplitWide = 24;
 // Longest context, in key tiles, of a PAIRED launch: up to two cells per CU, the same with
 // items known to be even, and above two.
 constexpr int kPairedTiles = 16;
@@ -1406,26 +1409,53 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   PrefillParams p = p0;
   p.positions_per_tile = prefill_positions_per_tile(p.group);
   const int cus = device_cu_count();
-  auto q_tiles = [&]() { return nothing ? 0 : (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile; };
-  p.num_q_tiles = q_tiles();
+  p.num_q_tiles = nothing ? 0 : (max_seqlen_q + p.positions_per_tile - 1) / p.positions_per_tile;
   // max_seqlen_k only sizes the cuts: a wrong value changes which items are
   // halved or split, never the result beyond rounding
   const int64_t kt_max = (std::max<int64_t>(max_seqlen_k, 0) + kBK - 1) / kBK;
   // Half the rows per item for a launch that leaves CUs idle: with 128 rows each SIMD runs
-  // one wave, and a key tile takes ~1.25 us instead of ~1.8, as do the item's first loads,
-  // merge and stores.  Where key halves want the idle CUs too, only up to 3/8 of the CUs
-  // (1/8 at d = 64, whose shorter tiles gain less).  Full -> half rows, d = 128: one prompt
-  // of 128 tokens, heads 16/8, 10.1 -> 8.2 us (8 items), 4 of 300 14.2 -> 12.4 (96), one of
-  // 1024 26.0 -> 22.9 (64), heads 4/1, 25.0 -> 21.5; 500 after 4096 cached 65 -> 50 (32); at
-  // 128 items one of 2048, heads 16/8, 37.5 -> 35.9, of 1024, 32/8, 27.5 -> 28.9, and of 500,
-  // 64/8, 20.6 -> 26.3.  d = 64, heads 14/2: 4 of 300 9.9 -> 8.2 (72, too short for key
-  // halves), one of 500 13.8 -> 13.0 (28), of 1024 18.9 -> 19.4 (58), of 2048 28.2 -> 48.8
-  // (114).
+  // one wave, and a key tile takes ~1.25 us instead of ~1.8, as do the item's first loads
+  // and stores.  The shorter tiles also move the line from which key halves pay for their
+  // merge: cut from 8 tiles on as whole items are, half-row items lost up to 24 tiles, to uncut
+  // ones and where CUs ran out to whole ones.  So contexts of up to kHalfRowsSplitWide tiles
+  // take them up to 3/8 of the CUs in whole items, uncut (cut above kHalfRowsSplit where they
+  // are few, or all of one or two sequences with room for the halves); longer ones where
+  // the items and the halves of those that are cut have a CU each, and the items take at most
+  // 1/2 of the CUs, or 5/8 below a GQA group of 8: beyond that a launch takes as long as
+  // with the heaviest items uncut (one prompt, heads 8/1, 126 -> 130 items: 35.0 -> 48.3 us;
+  // heads 4/1, 160 -> 168: 64.5 -> 79.1; why was not found).  At d = 64, whose tiles are
+  // shorter, up to 1/8 of the CUs in whole items.
+  // Attention.forward, whole rows -> half rows cut from 8 tiles on -> as here, us.  d = 128,
+  // heads 16/8: one prompt of 128 tokens 11.7 -> 8.9 -> 8.9, of 723 22.4 -> 20.1 -> 18.3, 2 of
+  // 512 after 256 cached 27.1 -> 24.3 -> 21.9, 723 after 2048 46.7 -> 38.8 -> 38.8; heads 8/1, 2 of
+  // 1500 after 256 cached 38.5 -> 58.5 -> 38.6 (whole), 3 of 1024 after 256 33.9 -> 48.7 ->
+  // 29.7; heads 32/8, 723 after 256 27.7 -> 36.5 -> 24.3; heads 4/1, 5120 78.1 -> 64.5 -> 64.5.
+  // d = 64, heads 14/2: one of 500 14.1 -> 13.4 -> 10.3, 4 of 300 10.3 -> 8.5 -> 8.6.
   const int64_t full_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
-  const int eighths = kt_max < kSplitMin ? 4 : (p.head_dim == 64 ? 1 : 3);
-  if (8 * full_items <= eighths * int64_t{cus} && p.positions_per_tile > 1) {
-    p.positions_per_tile /= 2;
-    p.num_q_tiles = q_tiles();
+  const int tpp = p.block_table ? p.block_size / kBK : 1;  // key tiles per page
+  const int64_t cut_tiles =  // an item of so many key tiles is cut where items are
+      std::max<int64_t>(std::max(kSplitMin, 2 * tpp), (kSplitNum * kt_max + kSplitDen - 1) / kSplitDen);
+  int split_min = kSplitMin;
+  if (!nothing && p.positions_per_tile > 1) {
+    const int half_ppt = p.positions_per_tile / 2;
+    const int half_tiles = (max_seqlen_q + half_ppt - 1) / half_ppt;
+    const int64_t pairs = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads;
+    // query tiles t whose keys, min(max_seqlen_k, (t + 1) half_ppt + cached), are too few for a cut
+    const int64_t uncut = std::max<int64_t>(0, ((cut_tiles - 1) * kBK - std::max(0, max_seqlen_k - max_seqlen_q)) / half_ppt);
+    const int64_t half_items = pairs * half_tiles;
+    const bool room = half_items + pairs * std::max<int64_t>(0, half_tiles - uncut) <= cus &&
+                      8 * half_items <= (p.group < 8 ? 5 : 4) * int64_t{cus};
+    const bool half = kt_max < kSplitMin             ? 2 * full_items <= cus
+                      : p.head_dim == 64             ? 8 * full_items <= cus
+                      : kt_max <= kHalfRowsSplitWide ? 8 * full_items <= 3 * int64_t{cus}
+                                                     : room;
+    if (half) {
+      p.positions_per_tile = half_ppt;
+      p.num_q_tiles = half_tiles;
+      const bool early = p.head_dim == 64 ? 8 * half_items <= cus
+                                          : 4 * half_items <= cus || (p.num_seqs <= 2 && room);
+      split_min = 1 + (early ? kHalfRowsSplit : kHalfRowsSplitWide);
+    }
   }
   // Persistent grid when there are enough items to balance; with at most two
   // per CU its table set-up (one more dependent global load and a few
@@ -1494,12 +1524,10 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   p.split_cus = cus;
   const int64_t pairs_split = kPrefillSplitSlots / p.num_kv_heads;  // at most this many pairs split
   // paged: the halves meet at a page boundary, so only items of at least two
-  // pages' tiles split (tpp tiles per page; pages of at most kSplitMaxPageTiles)
-  const int tpp = p.block_table ? p.block_size / kBK : 1;
-  if (p.split_ctl != nullptr && p.split_part != nullptr && max_items <= 2 * int64_t{cus} && kt_max >= kSplitMin &&
+  // pages' tiles split (pages of at most kSplitMaxPageTiles)
+  if (p.split_ctl != nullptr && p.split_part != nullptr && max_items <= 2 * int64_t{cus} && kt_max >= split_min &&
       pairs_split > 0 && tpp <= kSplitMaxPageTiles)
-    p.split_tiles = static_cast<int>(
-        std::max<int64_t>(std::max(kSplitMin, 2 * tpp), (kSplitNum * kt_max + kSplitDen - 1) / kSplitDen));
+    p.split_tiles = static_cast<int>(cut_tiles);
   // compact grid with key halving: every (sequence, tile) pair's position, one
   // more for each pair that may split
   const dim3 grid = p.split_tiles > 0

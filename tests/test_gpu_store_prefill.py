@@ -4,6 +4,8 @@ the same inputs, over the grids and head shapes that fuse, those that do not, an
 work item carries (past cu_seqlens_q's end, past max_seqlen_q)."""
 from __future__ import annotations
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -61,6 +63,40 @@ def test_matches_the_two_calls(dev, nh, nkv, d, lens):
         assert torch.equal(kc, rk) and torch.equal(vc, rv)
         # bit-identical but for key halves, whose merge takes the halves in order of arrival
         assert_attn_close(f32(o), f32(ro), what="output")
+
+
+SHORT_D64 = [1, 63, 64, 65, 300, 0, 777]  # 44 cells a sequence at heads 14/2, 13 key tiles
+
+
+@pytest.mark.parametrize("times", [1, 2, 3], ids=["key halves", "up to four per CU", "four per CU"])
+def test_two_workgroups_per_cu(dev, times):
+    """Head dim 64 with two workgroups per CU and the store in the launch: caches bit-identical to
+    store_kvcache and every output row against the oracle, with skipped slots, rows outside
+    cu_seqlens and positions past max_seqlen_q."""
+    from _helpers import assert_attn_close, f32, prefill_reference
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    lens = SHORT_D64 * times + [40] * (2 if times == 3 else 0)
+    cells = 2 * len(lens) * -(-max(lens) // 36)
+    lo, hi = ((cus, 2 * cus), (2 * cus, 3 * cus), (3 * cus, 4 * cus))[times - 1]
+    assert lo < cells <= hi and -(-max(lens) // 64) <= 16, "another grid"
+    c = _case(dev, lens, 14, 2, 64, seed=times)
+    c.slot_mapping[::5] = -1
+    c.slot_mapping[-1] = c.k_cache.shape[0] * c.k_cache.shape[1]
+    ref = prefill_reference(c)
+    _, rk, rv = _two_calls(c, c.k, c.v)
+    for _ in range(2):  # the workspace as the first call left it
+        o, kc, vc = _forward(c, c.k, c.v)
+        torch.cuda.synchronize()
+        assert torch.equal(kc, rk) and torch.equal(vc, rv)
+        assert_attn_close(f32(o), ref, what=f"{cells} cells")
+    _, kc, vc = _forward(c, c.k, c.v, max_q=max(lens) - 40)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, rk) and torch.equal(vc, rv)
+    c.cu_seqlens_q, c.cu_seqlens_k = (t[1:-1].contiguous() for t in (c.cu_seqlens_q, c.cu_seqlens_k))
+    assert cus < 2 * (len(lens) - 2) * -(-max(lens) // 36) or times == 1
+    _, kc, vc = _forward(c, c.k, c.v)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, rk) and torch.equal(vc, rv)
 
 
 @pytest.mark.parametrize("lens", [RAGGED, RAGGED * 9], ids=["direct", "persistent"])
@@ -164,3 +200,40 @@ def test_half_row_items(dev, nh, nkv, d, prefix, over):
         assert_attn_close(f32(o), prefill_reference(c), what=f"{seqs} sequences")
     rows = c.k_cache.view(-1, nkv, d)[c.slot_mapping.long()]
     assert torch.equal(rows, c.k)
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(16, 8, 128), (8, 1, 128), (14, 2, 64)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("keys", [16, 17, 24, 25], ids=lambda t: f"{t} tiles")
+@pytest.mark.parametrize("seqs", [1, 3, 9])
+def test_half_row_items_and_key_halves(dev, nh, nkv, d, fp8, keys, seqs):
+    """Half-row items on both sides of the context lengths from which they are cut in key halves
+    (one to nine sequences of 40 tokens behind a cached prefix, and the first alone long):
+    every row against the oracle."""
+    from _helpers import FP8_MAX_ABS, assert_attn_close, f32, prefill_reference
+    from nanovllm_amd import workloads as W
+    import nanovllm_amd as nva
+    if fp8 and d == 64:
+        pytest.skip("fp8 caches are read at head dim 128")
+    prefix = 64 * keys - 64
+    lens = [64] + [40] * (seqs - 1)
+    c = W.make_prefill_case(lens, nh, nkv, seqs * -(-(prefix + 64) // 64) + 2, prefix_len=prefix, block_size=64, head_dim=d,
+                            seed=keys + seqs, bulk_device=dev, shared_prefix=False)
+    layer = nva.Attention(nh, d, c.scale, nkv)
+    tol = {}
+    if fp8:
+        c.k_cache, layer.k_scale = W.quantize_cache_fp8(c.k_cache, extra=c.k)
+        c.v_cache, layer.v_scale = W.quantize_cache_fp8(c.v_cache, extra=c.v)
+        tol = dict(max_abs=FP8_MAX_ABS, mean_abs=FP8_MAX_ABS)
+    layer.k_cache, layer.v_cache = c.k_cache, c.v_cache
+    for _ in range(2):
+        nva.set_context(True, c.cu_seqlens_q, c.cu_seqlens_k, c.max_seqlen_q, c.max_seqlen_k, c.slot_mapping, None,
+                        c.block_tables)
+        o = layer(c.q, c.k, c.v).view(-1, nh, d)
+        nva.reset_context()
+        torch.cuda.synchronize()
+        ref = c
+        if fp8:  # the oracle reads the dequantised values
+            ref = SimpleNamespace(**{**vars(c), "k_cache": c.k_cache.float() * layer.k_scale[:, None],
+                                     "v_cache": c.v_cache.float() * layer.v_scale[:, None]})
+        assert_attn_close(f32(o), prefill_reference(ref), what=f"{keys} tiles", **tol)
