@@ -118,6 +118,7 @@ struct PrefillParams {
   // bf16 paged kernel's scalar registers: 0.5% slower at 8813 tokens after 1024 cached.)
   const float* k_scale;
   const float* v_scale;
+  int32_t rotate;             // direct grid at d 64: a query tile's (sequence, kv head) pairs start one XCD on
 };
 
 struct QKNormRopeParams {

@@ -1131,16 +1131,19 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // other's, where a single workgroup leaves them exposed; with fewer, the tighter
 // registers only cost (~10%: fewer operand reads in flight).  Up to two cells per CU the
 // alternative is this grid unpaired, where an item has a CU to itself and the lightest wait
-// for one; above two, the persistent grid, which evens out items of unequal work: two
-// heavy items on one CU set the length of a paired launch.  Attention.forward, heads 14/2, unpaired
-// (above 512 cells persistent) -> PAIRED, us.
-//   256 to 512 cells: 12 prompts of 100-1024 tokens 23.2 -> 18.9, 10 of 500 21.9 -> 17.8, 8 of
-//   128-1024 25.8 -> 21.6, 40 of 200 after 256 cached 28.6 -> 27.0; 12 of 350-700 21.4 -> 23.6;
-//   even items above 12 tiles, 5 of 1024 22.4 -> 26.7, 8 of 1024 28.9 -> 30.1; above 16 tiles,
-//   6 of 700-1400 27.0 -> 34.7, 4 of 2000 40.7 -> 47.6, one of 8000 127 -> 163.
-//   Up to 1024 cells: 24 of 300-700 36.0 -> 28.2, 32 of 400 after 1024 cached 87.5 -> 75.8; even,
-//   8 of 2000 86.4 -> 73.0, one of 10000 252 -> 222; above 28 tiles and not even, 4 of 500-4600
-//   100 -> 128, 8 of 600-2200 65.6 -> 70.4, 16 of 100-700 after 2048 cached 97 -> 112.
+// for one, or with idle CUs key halves; above two, the persistent grid, which evens out
+// items of unequal work.  On this grid those stay uneven twice over: two heavy items on a
+// CU, and with a multiple of 8 (sequence, kv head) pairs the long sequences on their own
+// XCDs (p.rotate spreads their tiles over all, at the price of the L2 that they share).
+// Attention.forward, heads 14/2, unpaired (above 512 cells persistent) -> PAIRED, us.
+//   257 to 512 cells, short: 12 prompts of 100-1024 tokens 23.2 -> 18.9, 10 of 500 21.9 -> 17.8, 40
+//   of 200 after 256 cached 28.6 -> 27.0; uneven with at most 9/8 CUs' real items, 4 of 253-2022
+//   tokens 46.0 -> 35.2 and 6 of 145-1163 28.0 -> 23.2; but above those counts 12 of 350-700 21.4 ->
+//   23.6, 6 of 700-1400 27.0 -> 34.7; even above 12 tiles, 5 of 1024 22.4 -> 26.7, one of 8000
+//   127 -> 163.
+//   Up to 1024 cells: 24 of 300-700 36.0 -> 28.2, 8 of 2000 86.4 -> 73.0, one of 10000 252 -> 222, 32
+//   of 400 after 1024 cached 87.5 -> 75.8; uneven in 8 pairs, 4 of 500-4600 100 -> 128 (rotated 94),
+//   16 of 100-700 after 2048 cached 97 -> 112.
 //   1344 cells, 24 prompts: 35 -> 42.
 template <int KV, int D, bool STORE, bool PAIRED = false>
 __global__ __launch_bounds__(64 * kWaves, PAIRED ? 4 : 2) void varlen_prefill_kernel(PrefillParams p) {
@@ -1161,8 +1164,12 @@ __global__ __launch_bounds__(64 * kWaves, PAIRED ? 4 : 2) void varlen_prefill_ke
     half = ci.half;
     pair = ci.pair;
   } else {
-    s = blockIdx.x / p.num_kv_heads;
-    kvh = blockIdx.x - s * p.num_kv_heads;
+    int x = blockIdx.x;
+    if constexpr (PAIRED) {
+      if (p.rotate) x = static_cast<int>((blockIdx.x + blockIdx.y) % gridDim.x);
+    }
+    s = x / p.num_kv_heads;
+    kvh = x - s * p.num_kv_heads;
     tile = p.num_q_tiles - 1 - static_cast<int>(blockIdx.y);
   }
   ItemDesc it = item_desc(p, p.cu_q, p.cu_k, s, kvh, tile);
@@ -1397,11 +1404,13 @@ constexpr int kSplitMaxPageTiles = 8;  // paged key halving for block sizes up t
 // Half-row items (launch_prefill): contexts above so many key tiles are cut in halves.
 constexpr int kHalfRowsSplit = 16;
 constexpr int kHalfRowsSplitWide = 24;
-// Longest context, in key tiles, of a PAIRED launch: up to two cells per CU, the same with
-// items known to be even, and above two.
-constexpr int kPairedTiles = 16;
+// Longest context, in key tiles, of a PAIRED launch of up to two cells per CU -- of items
+// known to be even, known not to be, unknown -- and of up to four, unknown.
 constexpr int kPairedTilesEven = 12;
+constexpr int kPairedTilesRagged = 8;
+constexpr int kPairedTiles = 16;
 constexpr int kPairedTilesTwo = 28;
+constexpr int kXcds = 8;  // workgroup id modulo this: the XCD
 
 hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seqlen_k, hipStream_t stream,
                           const StoreParams* store, int store_vec) {
@@ -1431,7 +1440,8 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   // 1500 after 256 cached 38.5 -> 58.5 -> 38.6 (whole), 3 of 1024 after 256 33.9 -> 48.7 ->
   // 29.7; heads 32/8, 723 after 256 27.7 -> 36.5 -> 24.3; heads 4/1, 5120 78.1 -> 64.5 -> 64.5.
   // d = 64, heads 14/2: one of 500 14.1 -> 13.4 -> 10.3, 4 of 300 10.3 -> 8.5 -> 8.6.
-  const int64_t full_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
+  const int64_t pairs = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads;
+  const int64_t full_items = pairs * p.num_q_tiles;
   const int tpp = p.block_table ? p.block_size / kBK : 1;  // key tiles per page
   const int64_t cut_tiles =  // an item of so many key tiles is cut where items are
       std::max<int64_t>(std::max(kSplitMin, 2 * tpp), (kSplitNum * kt_max + kSplitDen - 1) / kSplitDen);
@@ -1439,7 +1449,6 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   if (!nothing && p.positions_per_tile > 1) {
     const int half_ppt = p.positions_per_tile / 2;
     const int half_tiles = (max_seqlen_q + half_ppt - 1) / half_ppt;
-    const int64_t pairs = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads;
     // query tiles t whose keys, min(max_seqlen_k, (t + 1) half_ppt + cached), are too few for a cut
     const int64_t uncut = std::max<int64_t>(0, ((cut_tiles - 1) * kBK - std::max(0, max_seqlen_k - max_seqlen_q)) / half_ppt);
     const int64_t half_items = pairs * half_tiles;
@@ -1460,18 +1469,24 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   // Persistent grid when there are enough items to balance; with at most two
   // per CU its table set-up (one more dependent global load and a few
   // barriers) costs more than it saves (measured on config 2).
-  const int64_t max_items = static_cast<int64_t>(p.num_seqs) * p.num_kv_heads * p.num_q_tiles;
+  const int64_t max_items = pairs * p.num_q_tiles;
   // At D = 64 two workgroups fit a CU on the direct grid (see PAIRED, also for the figures
-  // that place these limits): above one cell per CU while the contexts are short, and above
-  // two, up to four, at any length where the items' work is known to be even -- one sequence,
-  // or fresh rows (the store's, the only count of them here) that fill 4/5 of num_seqs *
-  // max_seqlen_q.
-  const bool even = p.num_seqs == 1 || (store != nullptr && !p.block_table &&
-                                        5 * store->num_tokens >= 4 * int64_t{p.num_seqs} * max_seqlen_q);
-  const bool paired =
-      p.head_dim == 64 && max_items > cus &&
-      (max_items <= 2 * int64_t{cus} ? kt_max <= (even ? kPairedTilesEven : kPairedTiles)
-                                     : max_items <= 4 * int64_t{cus} && (even || kt_max <= kPairedTilesTwo));
+  // that place these lines).  How even the items' work is decides, and the launch knows it
+  // for fresh rows alone (from the store's count of them): `even` when they fill 17/20 of
+  // num_seqs * max_seqlen_q.
+  const bool counted = store != nullptr && !p.block_table;
+  const int64_t tokens = counted ? store->num_tokens : 0;
+  const bool even = p.num_seqs == 1 || (counted && 20 * tokens >= 17 * int64_t{p.num_seqs} * max_seqlen_q);
+  bool paired = false;
+  if (p.head_dim == 64 && max_items > cus && max_items <= 2 * int64_t{cus}) {
+    // real items, a half tile more per sequence than the rows fill
+    const int64_t real = p.num_kv_heads * tokens / p.positions_per_tile + pairs / 2;
+    paired = kt_max <= (even ? kPairedTilesEven : counted ? kPairedTilesRagged : kPairedTiles) ||
+             (counted && !even && 8 * real <= 9 * int64_t{cus});
+  } else if (p.head_dim == 64 && max_items > cus && max_items <= 4 * int64_t{cus}) {
+    paired = counted || even || pairs % kXcds != 0 || kt_max <= kPairedTilesTwo;
+    p.rotate = counted && !even && pairs % kXcds == 0;
+  }
   const bool persistent = p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles &&
                           max_items > 2 * int64_t{cus} && !paired;
   // one workgroup per CU (the ring takes most of a CU's LDS); the work queue
