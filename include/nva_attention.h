@@ -246,8 +246,10 @@ int nva_store_decode(const void* key, int64_t key_row_stride,
  * nva_store_kvcache of the new rows, then nva_decode, with the results of the two calls for any
  * slots (nva_store_decode without its conditions; same arguments).  In the spread mode the
  * store runs inside the decode launch: a wave that reads the slot of another row of the step
- * writes that row first.  Other plans launch the store before the decode, as do rows, queries
- * or an output that lie inside a cache.
+ * writes that row first, and of rows that share a valid slot the first one is stored and
+ * attended over.  Other plans launch the store before the decode, as do rows, queries or an
+ * output that lie inside a cache; which of several rows a slot then keeps is not defined, as in
+ * the two calls.
  */
 int nva_store_then_decode(const void* key, int64_t key_row_stride,
                           const void* value, int64_t value_row_stride,

@@ -660,26 +660,41 @@ __device__ __forceinline__ void store_row_wave(const DecodeParams& p, int kvh, i
     *reinterpret_cast<u32x4*>(dst) = x;
 }
 
+// Whether no earlier row of the step has row `row`'s slot.  store_exact stores only such rows:
+// of rows that share a slot the first one, so that every wave that writes a slot writes the
+// same bytes, whatever the order.
+__device__ __forceinline__ bool first_of_slot(const DecodeParams& p, int row, int slot) {
+  const int lane = threadIdx.x & 63;
+  for (int c0 = 0; c0 < row; c0 += 64) {
+    const int i = c0 + lane;
+    if (__builtin_amdgcn_ballot_w64(i < row && p.slot_mapping[min(i, row)] == slot) != 0) return false;
+  }
+  return true;
+}
+
 // store_exact: other rows of the step whose slots lie among this wave's keys [k_begin, k_end)
 // of sequence b (a padded row's slot that a live sequence owns; pages shared while being
 // written; none in an ordinary step).  The wave stores them itself before it reads,
 // so that it sees what a store before the launch would have shown it, whatever the
 // other waves have done; they write the same bytes.  Sequence b's own row at key ctx-1 is
-// left to the patch.  bt_row: lane j holds block-table entry j.  The check (the rows' slots
+// left to the patch.  bt_row: lane j holds block-table entry j; own: row b's slot.  Returns
+// first_of_slot of row b: otherwise an earlier row stands in its slot, and row b is neither
+// stored nor patched in.  The check (the rows' slots
 // against the wave's table entries, from registers) measures nothing; the store launch that
 // it saves took a decode of one sequence from 16.5 to 10.2 us, of 8 at d = 64 from 16.6 to
 // 10.3.
 template <bool FP8, int D>
-__device__ __forceinline__ void store_rows_read_here(const DecodeParams& p, int kvh, int b, int ctx, int k_begin, int k_end,
-                                                     int bt_row) {
+__device__ __forceinline__ bool store_rows_read_here(const DecodeParams& p, int kvh, int b, int ctx, int k_begin, int k_end,
+                                                     int bt_row, int own) {
   const int lane = threadIdx.x & 63;
   const int64_t num_slots = p.num_blocks * p.block_size;
-  bool any = false;
+  bool any = false, own_first = true;
   for (int c0 = 0; c0 < p.batch; c0 += 64) {
     const int i = c0 + lane;
     const int slot = i < p.batch ? p.slot_mapping[i] : -1;
     const int page = slot / p.block_size;
     const int off = slot - page * p.block_size;
+    if (__builtin_amdgcn_ballot_w64(i < b && slot == own) != 0) own_first = false;
     for (int e = k_begin / p.block_size; e * p.block_size < k_end; ++e) {
       const int key = e * p.block_size + off;
       const bool hit = slot >= 0 && slot < num_slots && page == __builtin_amdgcn_readlane(bt_row, e) && key >= k_begin &&
@@ -687,13 +702,16 @@ __device__ __forceinline__ void store_rows_read_here(const DecodeParams& p, int 
       for (uint64_t m = __builtin_amdgcn_ballot_w64(hit); m != 0; m &= m - 1) {
         const int L = static_cast<int>(__builtin_ctzll(m));
         const int64_t r = c0 + L;
+        const int at = __builtin_amdgcn_readlane(slot, L);
+        if (!first_of_slot(p, static_cast<int>(r), at)) continue;
         const uint16_t* src = (lane >= 32 ? p.new_v + r * p.new_v_stride : p.new_k + r * p.new_k_stride) + kvh * D;
-        store_row_wave<FP8, D>(p, kvh, __builtin_amdgcn_readlane(slot, L), ld16(src + 8 * (lane & (D / 8 - 1))));
+        store_row_wave<FP8, D>(p, kvh, at, ld16(src + 8 * (lane & (D / 8 - 1))));
         any = true;
       }
     }
   }
   if (any) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the stores are done before the reads
+  return own_first;
 }
 
 template <bool FP8, int D, bool STORE>
@@ -725,11 +743,12 @@ __global__ __launch_bounds__(64) void paged_decode_spread_kernel(DecodeParams p)
     // store-then-decode without waiting for the store.  An empty sequence's
     // rows are stored by the merge kernel, after every read of this launch.
     // With store_exact the result equals store-then-decode for any slots.
-    if (p.store_exact) store_rows_read_here<FP8, D>(p, kvh, b, ctx, k_begin, k_end, bt_row);
     const int64_t slot = __builtin_amdgcn_readfirstlane(p.slot_mapping[b]);
+    const bool own_first = !p.store_exact || store_rows_read_here<FP8, D>(p, kvh, b, ctx, k_begin, k_end, bt_row,
+                                                                          static_cast<int>(slot));
     const int holder = ctx > 0 ? (ctx - 1) / (32 * per) : -1;
     NewRow<FP8, D> nr;
-    const bool stores = r == holder && slot >= 0 && slot < static_cast<int64_t>(p.num_blocks) * p.block_size;
+    const bool stores = own_first && r == holder && slot >= 0 && slot < static_cast<int64_t>(p.num_blocks) * p.block_size;
     // lanes 0..D/8-1 store the key row, lanes 32.. the value row, 8 elements
     // each; the rows are loaded now and stored after the steps, so the store
     // never holds up this share's own loads
@@ -791,10 +810,12 @@ __global__ __launch_bounds__(64) void paged_decode_spread_kernel(DecodeParams p)
 // such a sequence, so the merge kernel -- stream-ordered after every read of
 // the decode launch -- stores them.  One wave: lanes 0..d/8-1 write the key
 // row, lanes 32..32+d/8-1 the value row, 8 elements each (fp8: quantised as
-// the store kernel does).  Slots outside the pool are skipped.
+// the store kernel does).  Slots outside the pool are skipped, and with store_exact those
+// of an earlier row.
 __device__ void store_empty_rows_wave(const DecodeParams& p, int b, int kvh, int lane) {
   const int64_t slot = p.slot_mapping[b];
   const int j = lane & 31;
+  if (p.store_exact && !first_of_slot(p, b, static_cast<int>(slot))) return;
   if (slot < 0 || slot >= p.num_blocks * p.block_size || 8 * j >= p.head_dim) return;
   const bool is_v = lane >= 32;
   const u32x4 x = ld16((is_v ? p.new_v + b * p.new_v_stride : p.new_k + b * p.new_k_stride) +
@@ -845,8 +866,8 @@ __global__ __launch_bounds__(64 * kShortSteps) void paged_decode_short_kernel(De
     u32x4 x = {0u, 0u, 0u, 0u};
     if constexpr (STORE) {
       const int64_t slot = __builtin_amdgcn_readfirstlane(p.slot_mapping[b]);
-      store_rows_read_here<FP8, D>(p, kvh, b, ctx, k_begin, k_end, bt_row);
-      stores = r == shares - 1 && slot >= 0 && slot < static_cast<int64_t>(p.num_blocks) * p.block_size;
+      stores = store_rows_read_here<FP8, D>(p, kvh, b, ctx, k_begin, k_end, bt_row, static_cast<int>(slot)) &&
+               r == shares - 1 && slot >= 0 && slot < static_cast<int64_t>(p.num_blocks) * p.block_size;
       if (stores) {
         const uint16_t* kin = p.new_k + b * p.new_k_stride + kvh * D;
         const uint16_t* vin = p.new_v + b * p.new_v_stride + kvh * D;

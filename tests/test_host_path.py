@@ -136,7 +136,7 @@ def test_decode_equals_store_then_decode(dev, monkeypatch, slots, B, nh, nkv, d,
         s[live] = (c.block_tables[live, 0] * 256).roll(-1)
     elif slots == "padding":  # rows without keys go to slots that live sequences read
         # (of more than one key: the row of a one-key sequence goes to that very slot, and which
-        # of two rows a slot keeps is not defined by the store either)
+        # of two rows a slot keeps is not defined by the store; test_rows_that_share_a_slot)
         empty = [b for b, n in enumerate(c.lengths) if n == 0]
         longer = [b for b in live if c.lengths[b] > 1]
         for i, b in enumerate(empty):
@@ -154,6 +154,46 @@ def test_decode_equals_store_then_decode(dev, monkeypatch, slots, B, nh, nkv, d,
     want, got, taken = _both(monkeypatch, run)
     assert taken == 1
     _same(want, got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [1, 4])  # one block: the short-table kernel
+@pytest.mark.parametrize("B,nh,nkv,d,fp8", [(3, 16, 8, 128, False), (10, 64, 8, 128, True), (32, 16, 8, 128, False),
+                                            (100, 14, 2, 64, False), (200, 4, 1, 128, False)])
+def test_rows_that_share_a_slot(dev, B, nh, nkv, d, fp8, width):
+    """Of rows that share a slot the spread mode stores the first, and every sequence attends over
+    what the caches then hold (bit-identical to the two calls with the later rows skipped)."""
+    import nanovllm_amd as nva
+    from nanovllm_amd import workloads as W
+    base = [1, 33, 0, 256, 0, 1, 31, 200, 0, 64]
+    lens = [base[i % len(base)] for i in range(B)]
+    c = W.make_decode_case(B, nh, nkv, 0, 0, B * width + 2, head_dim=d, fp8=fp8, seed=B, bulk_device=dev, lengths=lens,
+                           table_width=width)
+    last = [int(c.block_tables[b, (n - 1) // 256]) * 256 + (n - 1) % 256 if n else -1 for b, n in enumerate(lens)]
+    s = list(last)
+    for b in range(1, B):
+        if b % 3 == 2 or lens[b] == 0:  # an earlier or a later row's slot, or its sequence's first key
+            o = (b * 7 + 1) % B
+            s[b] = last[o] if b % 2 else int(c.block_tables[o, 0]) * 256
+    if lens[0] == 1 and B > 2:
+        s[2] = s[0]  # a row without keys against the only key of a sequence
+    seen, first = set(), []
+    for x in s:
+        first.append(-1 if x in seen else x)
+        seen.add(x)
+    assert any(x != y for x, y in zip(s, first))
+
+    def slots(x):
+        return torch.tensor(x, dtype=torch.int32, device=dev)
+    layer = _layer(c, c.k_cache.clone(), c.v_cache.clone(), (c.k_scale, c.v_scale))
+    nva.set_context(False, slot_mapping=slots(s), context_lens=c.context_lens, block_tables=c.block_tables)
+    o = layer(c.q, c.k_new, c.v_new).view(B, nh, d)
+    nva.reset_context()
+    nva.store_kvcache(c.k_new, c.v_new, c.k_cache, c.v_cache, slots(first), c.k_scale, c.v_scale)
+    two = nva.flash_attn_with_kvcache(c.q.unsqueeze(1), c.k_cache, c.v_cache, c.context_lens, c.block_tables,
+                                      softmax_scale=c.scale, k_scale=c.k_scale, v_scale=c.v_scale)
+    torch.cuda.synchronize()
+    _same((two[:, 0], c.k_cache, c.v_cache), (o, layer.k_cache, layer.v_cache))
 
 
 @pytest.mark.gpu
