@@ -78,12 +78,21 @@ def _compile(src: Path, verbose: bool) -> Path:
 
 
 def _build_host(verbose: bool) -> None:
-    """The host module, linked against the installed torch (its ABI)."""
-    import torch
-    root = Path(torch.__file__).resolve().parent
+    """The host module, linked against the installed torch (its ABI).  It saves host time only:
+    without a C++ compiler or torch's headers it is left out, and the calls run in Python."""
+    HOST_LIB.unlink(missing_ok=True)
+    try:
+        import torch
+        root = Path(torch.__file__).resolve().parent
+    except ImportError:
+        root = None
+    cxx = shutil.which(os.environ.get("CXX", "g++"))
+    if cxx is None or root is None or not (root / "include" / "ATen" / "ATen.h").exists():
+        print(f"{HOST_LIB.name} left out: no C++ compiler or no torch headers", flush=True)
+        return
     rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
     tmp = HOST_LIB.with_suffix(".so.tmp")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{INCLUDE}", "-isystem", str(root / "include"),
            "-isystem", str(root / "include" / "torch" / "csrc" / "api" / "include"), "-isystem", str(rocm / "include"),

@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstring>
 
@@ -313,4 +314,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_nva_host", nullptr, -1, methods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__nva_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__nva_host() {
+  PyObject* m = PyModule_Create(&module);
+  // the torch whose C++ ABI this was compiled against; the loader compares it
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -9,6 +9,7 @@ import ctypes
 import importlib.util
 import os
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libnva_attn.so"
@@ -185,18 +186,47 @@ _HOST_ENTRIES = ("nva_store_kvcache", "nva_prefill", "nva_prefill_fp8", "nva_sto
 _host = None
 
 
+class _NoHost:
+    """Stands in for a host module that cannot be used: takes no call, so every call runs the
+    general Python path over the same library."""
+
+    @staticmethod
+    def attention(*args):
+        return None
+
+    @staticmethod
+    def qk_norm_rope(*args):
+        return None
+
+
+def _load_host():
+    import torch
+    lib = load()
+    if not HOST_PATH.exists():
+        raise ImportError("not built: run `python nano-vllm_amd/build.py`")
+    spec = importlib.util.spec_from_file_location("_nva_host", HOST_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    built = getattr(mod, "torch_version", "of another version")
+    if built != torch.__version__.split("+")[0]:
+        raise ImportError(f"built for torch {built}, this is {torch.__version__}")
+    mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES))
+    return mod
+
+
 def host():
-    """The native form of the per-step calls (csrc/host/nva_host.cpp), bound to the loaded library."""
+    """The native form of the per-step calls (csrc/host/nva_host.cpp), bound to the loaded library.
+    It only saves host time: where it is missing or was built for another torch, a warning
+    says so once and the calls run the general Python path."""
     global _host
     if _host is None:
-        lib = load()
-        if not HOST_PATH.exists():
-            raise RuntimeError(f"{HOST_PATH} is not built: run `python nano-vllm_amd/build.py`")
-        spec = importlib.util.spec_from_file_location("_nva_host", HOST_PATH)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
-        mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES))
-        _host = mod
+        try:
+            _host = _load_host()
+        except ImportError as e:
+            load()  # a missing library still raises
+            warnings.warn(f"{HOST_PATH} is not used ({e}): Attention.forward and qk_norm_rope take 20 us more a call",
+                          RuntimeWarning, stacklevel=3)
+            _host = _NoHost
     return _host
 
 

@@ -43,6 +43,21 @@ class _Spy:
         return o
 
 
+def test_host_module_missing(monkeypatch, tmp_path):
+    """Without the host module, and with one built for another torch, the calls run in Python."""
+    from nanovllm_amd import _capi
+    assert _capi.host().torch_version == torch.__version__.split("+")[0]
+    for path, version in ((tmp_path / "_nva_host.so", torch.__version__), (_capi.HOST_PATH, "1.0.0")):
+        with monkeypatch.context() as m:
+            m.setattr(_capi, "_host", None)
+            m.setattr(_capi, "HOST_PATH", path)
+            m.setattr(torch, "__version__", version)
+            with pytest.warns(RuntimeWarning, match="is not used"):
+                host = _capi.host()
+            assert host.attention(1, 2) is None and host.qk_norm_rope(1) is None
+            assert _capi.host() is host
+
+
 def _layer(c, k_cache, v_cache, scales=(None, None)):
     import nanovllm_amd as nva
     layer = nva.Attention(c.num_heads, c.head_dim, c.scale, c.num_kv_heads)
