@@ -105,13 +105,16 @@ class DecodeGraphs:
     def _stage(self, size: int, q, k, v, slot_mapping, context_lens, block_tables) -> bool:
         """The static buffers' rows up to `size` (all that the graph of that size reads)
         written by one launch (nva_stage_decode).  False, with nothing done, for inputs
-        that the launch does not take as they are -- other types or devices (or another
-        current device), rows that are
-        not contiguous and 16-byte aligned, other shapes -- which the tensor copies of
-        run() convert, or reject."""
+        that the launch does not take as they are -- tensors that are not what their memory
+        holds (subclasses, negated views), other types or devices (or another current
+        device), rows that are not contiguous and 16-byte aligned, other shapes -- which the
+        tensor copies of run() convert, or reject."""
         bs, dev = q.shape[0], self.q.device
         if bs == 0 or torch.cuda.current_device() != dev.index:
             return False
+        for x in (q, k, v, slot_mapping, context_lens, block_tables):
+            if type(x) is not torch.Tensor or x.is_neg():
+                return False
         rows = []
         for x, buf in ((q, self.q), (k, self.k), (v, self.v)):
             if x.dtype != torch.bfloat16 or x.device != dev or x.shape[0] != bs or x.numel() != bs * buf.shape[1]:

@@ -174,7 +174,7 @@ def test_fp8_cache_replay_matches_oracle(dev):
 
 
 @pytest.mark.parametrize("bs", [1, 5, 16])
-def test_staged_inputs_equal_the_tensor_copies(dev, bs):
+def test_staged_inputs_equal_the_tensor_copies(dev, monkeypatch, bs):
     """The static buffers as the one-launch staging writes them (rows up to the graph's size)
     equal the fills and copies; inputs it does not take (int64 slots, unaligned or
     transposed rows) go through the copies with the same replayed result."""
@@ -194,8 +194,20 @@ def test_staged_inputs_equal_the_tensor_copies(dev, bs):
         assert torch.equal(buf[:bs], rows) and bool((buf[bs:size] == fill).all())
     assert torch.equal(graphs.block_tables[:bs, :3], bt) and not bool(graphs.block_tables[:bs, 3:].any())
     assert not bool(graphs.block_tables[bs:size].any())
+    for buf in (graphs.q, graphs.k, graphs.v, graphs.slot_mapping, graphs.context_lens, graphs.block_tables):
+        assert bool((buf[size:] == 7).all())  # the one launch leaves the rows past the graph's size
+    staged = []
+    real = graphs._stage
+    monkeypatch.setattr(graphs, "_stage", lambda *a: staged.append(real(*a)) or staged[-1])
+    assert torch.equal(torch.stack(graphs.run(q, k, v, slots, ctx, bt)), want) and staged == [True]
     odd = torch.empty(bs, D2 + 1, dtype=torch.bfloat16, device=dev)[:, 1:]
     odd.copy_(q)
-    for args in ((q, k, v, slots.long(), ctx, bt), (odd, k, v, slots, ctx, bt),
-                 (q.t().contiguous().t(), k, v, slots, ctx, bt), (q.float(), k, v, slots, ctx, bt)):
+
+    class Sub(torch.Tensor):
+        pass
+
+    for args in ((torch._neg_view(-q), k, v, slots, ctx, bt), (q, k.as_subclass(Sub), v, slots, ctx, bt),
+                 (q, k, v, slots.long(), ctx, bt), (odd, k, v, slots, ctx, bt),
+                 (torch.cat([q, q]).t().contiguous().t()[:bs], k, v, slots, ctx, bt), (q.float(), k, v, slots, ctx, bt)):
         assert torch.equal(torch.stack(graphs.run(*args)), want)
+        assert staged.pop() is False
