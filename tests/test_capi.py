@@ -288,3 +288,144 @@ def test_decode_noalloc_refuses_above_its_scratch(lib):
     rc = lib.nva_decode_noalloc(A, 128, B, C, 0, None, None, 100, A, A, 64, 64, 256, 4, 16, 8, 96, 0.1, 0,
                                 B, 128, None)
     assert rc == _capi.NVA_ERR_UNSUPPORTED
+
+
+def prefill_fp8(lib, **kw):
+    args = dict(q=A, q_row_stride=2048, k_cache=B, v_cache=C, k_scale=A + 0x8000, v_scale=A + 0x8100,
+                block_table=A + 0x9800, bt_row_stride=8, max_blocks=8, block_size=256, num_blocks=64, cu_q=A + 0x9000,
+                cu_k=A + 0xA000, num_seqs=2, max_seqlen_q=100, max_seqlen_k=500, num_heads=16, num_kv_heads=8,
+                head_dim=128, scale=0.088, out=C + 0x200000, out_row_stride=2048, workspace=None, workspace_bytes=0,
+                stream=None)
+    args.update(kw)
+    return lib.nva_prefill_fp8(*args.values())
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(head_dim=64), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(block_table=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k_scale=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(v_scale=A + 0x8102), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(block_size=96), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(bt_row_stride=4), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(num_heads=12), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(q_row_stride=1024), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k_cache=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k_cache=B + 8), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(scale=0.0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(workspace=A + 0x100000, workspace_bytes=128), _capi.NVA_ERR_INVALID_ARGUMENT),
+])
+def test_prefill_fp8_rejects(lib, kw, code):
+    assert prefill_fp8(lib, **kw) == code
+    assert lib.nva_last_error().decode()
+
+
+def test_prefill_fp8_empty_is_noop(lib):
+    assert prefill_fp8(lib, num_seqs=0, q=None, k_scale=None, block_table=None) == _capi.NVA_OK
+    assert prefill_fp8(lib, max_seqlen_q=0) == _capi.NVA_OK
+
+
+def store_prefill(lib, **kw):
+    args = dict(k_cache=C + 0x400000, v_cache=C + 0x800000, num_slots=4096, slot_mapping=A + 0x8000, num_tokens=200,
+                cache_dtype=0, k_scale=None, v_scale=None, q=A, q_row_stride=2048, num_queries=200, k=B,
+                k_row_stride=1024, v=B + 0x80000, v_row_stride=1024, cu_q=A + 0x9000, cu_k=A + 0xA000, num_seqs=2,
+                max_seqlen_q=100, max_seqlen_k=100, num_heads=16, num_kv_heads=8, head_dim=128, scale=0.088,
+                out=C + 0x2000000, out_row_stride=2048, workspace=None, workspace_bytes=0, stream=None)
+    args.update(kw)
+    return lib.nva_store_prefill(*args.values())
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(num_tokens=-1), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(num_slots=0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(cache_dtype=7), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(cache_dtype=1), _capi.NVA_ERR_INVALID_ARGUMENT),           # fp8 without scales
+    (dict(slot_mapping=A + 0x8002), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k_row_stride=1000), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(q=None), _capi.NVA_ERR_INVALID_ARGUMENT),                  # the attention's half
+    (dict(q_row_stride=1024), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(num_heads=12), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(scale=0.0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(workspace=A + 0x100000, workspace_bytes=128), _capi.NVA_ERR_INVALID_ARGUMENT),
+])
+def test_store_prefill_rejects(lib, kw, code):
+    """Both halves are validated before any launch (nothing lies inside the caches here)."""
+    assert store_prefill(lib, **kw) == code
+    assert lib.nva_last_error().decode()
+
+
+def test_store_prefill_empty_is_noop(lib):
+    """No tokens and no sequences: neither half has anything to launch."""
+    assert store_prefill(lib, num_tokens=0, num_queries=0, num_seqs=0, q=None) == _capi.NVA_OK
+    assert store_prefill(lib, num_tokens=0, num_queries=0, max_seqlen_q=0) == _capi.NVA_OK
+
+
+def store_then_decode(lib, **kw):
+    st = dict(key=A + 0x100000, key_row_stride=1024, value=A + 0x180000, value_row_stride=1024,
+              slot_mapping=A + 0xB000)
+    dec = dict(q=A, q_row_stride=2048, k_cache=0x10000000, v_cache=0x80000000, kv_dtype=0, k_scale=None, v_scale=None,
+               num_blocks=2048, seqlens=A + 0x9000, block_table=A + 0xA000, bt_row_stride=8, max_blocks=8,
+               block_size=256, batch=256, num_heads=16, num_kv_heads=8, head_dim=128, scale=0.088,
+               num_splits=0, out=C + 0x200000, out_row_stride=2048, workspace=None, workspace_bytes=0,
+               stream=None)
+    for d in (st, dec):
+        for k in list(kw):
+            if k in d:
+                d[k] = kw.pop(k)
+    assert not kw, kw
+    return lib.nva_store_then_decode(*st.values(), *dec.values())
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(key_row_stride=512), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(key=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(slot_mapping=A + 0xB002), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(kv_dtype=1), _capi.NVA_ERR_INVALID_ARGUMENT),              # fp8 without scales
+    (dict(num_blocks=0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(block_size=0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(batch=-1), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(head_dim=96, key_row_stride=768, value_row_stride=768), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(workspace=A, workspace_bytes=16), _capi.NVA_ERR_WORKSPACE),
+    (dict(out=C + 8), _capi.NVA_ERR_UNSUPPORTED),
+])
+def test_store_then_decode_rejects(lib, kw, code):
+    """Both halves are validated before any launch (nothing lies inside the caches here)."""
+    assert store_then_decode(lib, **kw) == code
+    assert lib.nva_last_error().decode()
+
+
+def test_store_then_decode_batch_zero_is_noop(lib):
+    assert store_then_decode(lib, batch=0) == _capi.NVA_OK
+
+
+def stage_decode(lib, **kw):
+    args = dict(q=A, q_row_stride=4096, k=B, k_row_stride=4096, v=C, v_row_stride=4096, slot_mapping=A + 0x8000,
+                context_lens=A + 0x9000, block_table=A + 0xA000, bt_row_stride=3, bt_width=3, live_rows=5, q_elems=2048,
+                kv_elems=1024, q_out=A + 0x100000, k_out=A + 0x200000, v_out=A + 0x300000, slots_out=A + 0x400000,
+                lens_out=A + 0x400100, table_out=A + 0x400200, out_width=16, rows=8, pad_slot=-1, stream=None)
+    args.update(kw)
+    return lib.nva_stage_decode(*args.values())
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(live_rows=-1), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(rows=4), _capi.NVA_ERR_INVALID_ARGUMENT),                  # fewer than the live ones
+    (dict(q_elems=0), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(out_width=2), _capi.NVA_ERR_INVALID_ARGUMENT),             # narrower than the given table
+    (dict(q=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(block_table=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(lens_out=None), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(k_row_stride=1016), _capi.NVA_ERR_INVALID_ARGUMENT),       # < kv_elems
+    (dict(bt_row_stride=2), _capi.NVA_ERR_INVALID_ARGUMENT),
+    (dict(v=C + 8), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(q_row_stride=4100), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(kv_elems=1020, q_elems=2048), _capi.NVA_ERR_UNSUPPORTED),
+    (dict(slot_mapping=A + 0x8002), _capi.NVA_ERR_INVALID_ARGUMENT),
+])
+def test_stage_decode_rejects(lib, kw, code):
+    assert stage_decode(lib, **kw) == code
+    assert lib.nva_last_error().decode()
+
+
+def test_stage_decode_no_rows_is_noop(lib):
+    assert stage_decode(lib, rows=0, live_rows=0, q=None, q_out=None) == _capi.NVA_OK

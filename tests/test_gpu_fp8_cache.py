@@ -253,3 +253,20 @@ def test_fp8_prefill_through_the_gather(dev, monkeypatch, d, bs, limit):
     assert_attn_close(_fp8_prefill(c, ks, vs), prefill_reference(ref), max_abs=FP8_MAX_ABS, mean_abs=FP8_MAX_ABS,
                       what="fp8 gather")
     assert A._GATHER_BUFFERS
+
+
+@pytest.mark.parametrize("nh,nkv,lens,prefix", [
+    (32, 8, [100, 700, 33], [512, 256, 768]), (4, 1, [206] * 6, [256] * 6), (64, 8, [300], [512])])
+def test_fp8_in_place_is_no_less_precise(dev, monkeypatch, nh, nkv, lens, prefix):
+    """Converting the pages as they are staged rounds nothing (the scales are applied in float32),
+    where the gather rounds every scaled row to bf16: its error against float64 is the
+    smaller one of the two."""
+    from _helpers import prefill_reference
+    from nanovllm_amd.layers import attention as A
+    c, ks, vs, ref = _fp8_prefill_case(dev, lens, nh, nkv, 128, 256, prefix, seed=nh)
+    want = prefill_reference(ref, dtype=np.float64)
+    err = {}
+    for name, limit in (("in place", 4096), ("gather", 0)):
+        monkeypatch.setattr(A, "_FP8_IN_PLACE_TOKENS", limit)
+        err[name] = np.linalg.norm(_fp8_prefill(c, ks, vs).astype(np.float64) - want) / np.linalg.norm(want)
+    assert err["in place"] < err["gather"] < 0.01, err

@@ -300,10 +300,65 @@ def test_other_forms_are_left_to_the_general_path(dev):
         assert call(**kw) is None, kw.keys()
     with Mode():
         assert call() is None
+    with torch.device("cpu"):  # a function mode (as torch.set_default_device installs)
+        assert call() is None
+    assert call() is not None
     assert torch.func.vmap(lambda x: (call(q=x) is None) * x.sum())(c.q.unsqueeze(0)) is not None
     seen = []
     torch.func.vmap(lambda x: (seen.append(call(q=x)), x)[1])(c.q.unsqueeze(0))
     assert seen == [None]
+
+
+@pytest.mark.gpu
+def test_streams_and_threads(dev):
+    """Native decodes and prefills on streams of their own, from two threads at once, equal those
+    on the default stream (each stream has its own prefill workspace)."""
+    import threading
+
+    import nanovllm_amd as nva
+    from nanovllm_amd import _capi
+    from nanovllm_amd import workloads as W
+    from nanovllm_amd.layers import attention as A
+    host = _capi.host()
+    dec = [_decode_inputs(dev, 40, 16, 8, 128, False, seed=i) for i in range(2)]
+    pre = [W.make_prefill_case([900, 300 + i, 40], 16, 8, 12, seed=i, bulk_device=dev) for i in range(2)]
+
+    def both(i):
+        c, p = dec[i], pre[i]
+        kc, vc, pk, pv = c.k_cache.clone(), c.v_cache.clone(), p.k_cache.clone(), p.v_cache.clone()
+        stream = torch.cuda.current_stream(dev)
+        nva.flash_attn_varlen_func(p.q, p.k, p.v, p.max_seqlen_q, p.cu_seqlens_q, p.max_seqlen_k, p.cu_seqlens_k, p.scale)
+        a = host.attention(c.q, c.k_new, c.v_new, kc, vc, None, None, 16, 8, 128, c.scale, False, False, None, None, 0, 0,
+                           c.slot_mapping, c.context_lens, c.block_tables, {}, 4096)
+        b = host.attention(p.q, p.k, p.v, pk, pv, None, None, 16, 8, 128, p.scale, False, True, p.cu_seqlens_q,
+                           p.cu_seqlens_k, p.max_seqlen_q, p.max_seqlen_k, p.slot_mapping, None, None,
+                           A._PREFILL_WORKSPACES, 4096)
+        assert a is not None and b is not None
+        stream.synchronize()
+        return a, kc, vc, pk, pv, b
+
+    want = [both(i) for i in range(2)]
+    torch.cuda.synchronize()
+    got, errors = [None, None], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream(dev)):
+                for _ in range(5):
+                    got[i] = both(i)
+        except Exception as e:  # a thread's exception would be lost
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for w, g in zip(want, got):
+        _same(w[:5], g[:5])
+        # key halves merge in order of arrival: the prefill's outputs to rounding
+        assert float((w[5].float() - g[5].float()).abs().max()) < 2e-2
 
 
 def test_host_tensors_are_left_to_the_general_path():
