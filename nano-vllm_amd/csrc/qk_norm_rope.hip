@@ -5,13 +5,13 @@
 //   q, k = rotary_emb(positions, q, k)           rotary_embedding.py:6-17, 37-55
 // With no norm weights it is the rotary embedding alone (Qwen2, qwen2.py:91-92).
 //
-// A wave takes kChunks x 64/LPR head rows of one token, LPR = D/16 lanes per row.
-// Lane j of a row holds 8 consecutive elements of each half of the head dimension,
+// A wave takes 64/LPR head rows of one token (LPR = D/16 lanes per row), or kChunks times as
+// many.  Lane j of a row holds 8 consecutive elements of each half of the head dimension,
 // [8 j, 8 j + 8) and [D/2 + 8 j, ...), so the rotation pairs (i, i + D/2) are
 // lane-local and only the sum of squares crosses lanes (xor shuffles over LPR
 // lanes).
 //
-// What bounds it: HBM (each row is read once and written once).  So a lane moves 16
+// What bounds a large launch: HBM (each row is read once and written once).  So a lane moves 16
 // bytes per access and issues all its rows' loads before any of them is used (4 KiB in
 // flight per wave at D = 128), the token's cos/sin row is loaded once for all of a
 // wave's heads (per head it is twice the bytes of the row itself, through L1), and no
@@ -23,15 +23,19 @@
 // a decode of 128 rows 34.3 -> 34.0 us (producer and attention together, plain against
 // non-temporal).
 //
+// A small launch (up to kSmallRows rows: every decode step) is bound by one wave's latency:
+// one chunk per wave, half the code, and the norm weights loaded with the rows instead of
+// after the reduction that needs them.  Captured, heads 16/8 with norm, 2 chunks -> 1: 1 token
+// 3.0 -> 2.5 us, 33 3.4 -> 2.75, 256 3.5 -> 2.9; heads 32/8, 256 tokens 3.7 -> 3.3 (10240
+// rows), 512 4.0 -> 4.2 (20480), hence the line.
+//
 // Arithmetic follows the reference's eager op sequence, rounding where it
 // rounds: fp32 x, mean of squares, x * rsqrt(mean + eps) rounded to bf16, times
 // the bf16 weight rounded to bf16; then fp32 x1*cos - x2*sin and x2*cos + x1*sin
 // with every product and sum rounded separately (no FMA contraction), rounded
 // to bf16.  The sum of squares runs in this kernel's order (a lane's squares,
 // then a butterfly over the row's lanes), which can move the mean by an fp32 ulp against
-// torch's reduction and so, rarely, an output by one bf16 ulp.  Memory-bound:
-// each row is read once and written once; the cos/sin row of a token is shared
-// by its heads through the caches.
+// torch's reduction and so, rarely, an output by one bf16 ulp.
 #include "nva_common.h"
 #include "nva_kernels.h"
 
@@ -40,6 +44,7 @@ namespace nva {
 namespace {
 
 constexpr int kChunks = 2;         // head chunks of a token that one wave takes
+constexpr int64_t kSmallRows = 16384;  // head rows up to which a launch is bound by latency
 constexpr int kTokensPerGroup = 4;  // waves per workgroup, one token each
 constexpr int64_t kMaxGroups = int64_t{1} << 22;  // tokens beyond 4 per workgroup: further rounds of the grid
 
@@ -51,10 +56,12 @@ __device__ __forceinline__ u32x4 load8(const uint16_t* p) {
   const uint32_t* w = reinterpret_cast<const uint32_t*>(p);
   return u32x4{w[0], w[1], w[2], w[3]};
 }
-template <bool WIDE>
+template <bool WIDE, bool NT>
 __device__ __forceinline__ void store8(uint16_t* p, u32x4 v) {
-  if constexpr (WIDE) {
+  if constexpr (WIDE && NT) {
     __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+  } else if constexpr (WIDE) {
+    st16(p, v);
   } else {
     uint32_t* w = reinterpret_cast<uint32_t*>(p);
 #pragma unroll
@@ -94,7 +101,7 @@ __device__ __forceinline__ void round8(float (&f)[8]) {
 
 }  // namespace
 
-template <int D, bool WIDE>
+template <int D, bool WIDE, int CHUNKS, bool NT>
 __global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNormRopeParams p) {
   // every product and sum rounds on its own, as the reference's separate ops do:
   // no FMA contraction anywhere in this function
@@ -104,17 +111,17 @@ __global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNo
   const int lane = threadIdx.x & 63;
   const int j = lane & (LPR - 1);
   const int heads = p.num_heads + p.num_kv_heads;
-  const int h0 = static_cast<int>(blockIdx.y) * kChunks * RPW;
+  const int h0 = static_cast<int>(blockIdx.y) * CHUNKS * RPW;
   const int64_t step = static_cast<int64_t>(gridDim.x) * kTokensPerGroup;
   for (int64_t t = static_cast<int64_t>(blockIdx.x) * kTokensPerGroup +
                    __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
        t < p.num_tokens; t += step) {
     int64_t pos = p.positions[t];
-    const uint16_t* src[kChunks];
-    uint16_t* dst[kChunks];
-    u32x4 lo[kChunks], hi[kChunks];
+    const uint16_t* src[CHUNKS];
+    uint16_t* dst[CHUNKS];
+    u32x4 lo[CHUNKS], hi[CHUNKS];
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
+    for (int c = 0; c < CHUNKS; ++c) {
       const int hh = h0 + c * RPW + lane / LPR;
       const bool is_q = hh < p.num_heads;
       src[c] = is_q ? p.q + t * p.q_row_stride + hh * D : p.k + t * p.k_row_stride + (hh - p.num_heads) * D;
@@ -126,13 +133,21 @@ __global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNo
         hi[c] = load8<WIDE>(src[c] + D / 2 + 8 * j);
       }
     }
+    u32x4 wlo = {0u, 0u, 0u, 0u}, whi = {0u, 0u, 0u, 0u};
+    if constexpr (CHUNKS == 1) {
+      if (p.q_weight) {
+        const uint16_t* wt = h0 + lane / LPR < p.num_heads ? p.q_weight : p.k_weight;
+        wlo = load8<WIDE>(wt + 8 * j);
+        whi = load8<WIDE>(wt + D / 2 + 8 * j);
+      }
+    }
     // cache row = [cos(D/2) | sin(D/2)] of the clamped position
     pos = pos < 0 ? 0 : (pos >= p.max_position ? p.max_position - 1 : pos);
     float cs[8], sn[8];
     load8f<WIDE>(p.cos_sin + pos * D + 8 * j, cs);
     load8f<WIDE>(p.cos_sin + pos * D + D / 2 + 8 * j, sn);
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
+    for (int c = 0; c < CHUNKS; ++c) {
       if (h0 + c * RPW >= heads) break;  // uniform: the whole chunk lies past the last head
       const int hh = h0 + c * RPW + lane / LPR;
       float x1[8], x2[8];
@@ -145,10 +160,14 @@ __global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNo
 #pragma unroll
         for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, LPR);
         const float r = rsqrtf(ss / static_cast<float>(D) + p.eps);
-        const uint16_t* wt = hh < p.num_heads ? p.q_weight : p.k_weight;
+        if constexpr (CHUNKS > 1) {
+          const uint16_t* wt = hh < p.num_heads ? p.q_weight : p.k_weight;
+          wlo = load8<WIDE>(wt + 8 * j);
+          whi = load8<WIDE>(wt + D / 2 + 8 * j);
+        }
         float w1[8], w2[8];
-        unpack8(load8<WIDE>(wt + 8 * j), w1);
-        unpack8(load8<WIDE>(wt + D / 2 + 8 * j), w2);
+        unpack8(wlo, w1);
+        unpack8(whi, w2);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           x1[e] *= r;
@@ -178,8 +197,8 @@ __global__ __launch_bounds__(64 * kTokensPerGroup) void qk_norm_rope_kernel(QKNo
         o2[w] = pack_bf16x2(y2[0], y2[1]);
       }
       if (hh < heads) {
-        store8<WIDE>(dst[c] + 8 * j, o1);
-        store8<WIDE>(dst[c] + D / 2 + 8 * j, o2);
+        store8<WIDE, NT>(dst[c] + 8 * j, o1);
+        store8<WIDE, NT>(dst[c] + D / 2 + 8 * j, o2);
       }
     }
   }
@@ -196,23 +215,26 @@ static bool rows_aligned16(const QKNormRopeParams& p) {
 hipError_t launch_qk_norm_rope(const QKNormRopeParams& p, hipStream_t stream) {
   const int heads = p.num_heads + p.num_kv_heads;
   if (p.num_tokens <= 0 || heads <= 0) return hipSuccess;
-  const int per_wave = kChunks * 64 / (p.head_dim / 16);  // heads
+  const int chunk = 64 / (p.head_dim / 16);  // heads
+  const bool small = p.num_tokens * heads <= kSmallRows;
+  const int per_wave = small ? chunk : kChunks * chunk;
   const int64_t groups = (p.num_tokens + kTokensPerGroup - 1) / kTokensPerGroup;
   const dim3 grid(static_cast<unsigned>(groups < kMaxGroups ? groups : kMaxGroups),
                   static_cast<unsigned>((heads + per_wave - 1) / per_wave));
   const dim3 block(64 * kTokensPerGroup);
   const bool wide = rows_aligned16(p);
-  if (p.head_dim == 128) {
-    if (wide)
-      hipLaunchKernelGGL((qk_norm_rope_kernel<128, true>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((qk_norm_rope_kernel<128, false>), grid, block, 0, stream, p);
-  } else {
-    if (wide)
-      hipLaunchKernelGGL((qk_norm_rope_kernel<64, true>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((qk_norm_rope_kernel<64, false>), grid, block, 0, stream, p);
-  }
+#define NVA_ROPE(DD, WD, CH, NT) hipLaunchKernelGGL((qk_norm_rope_kernel<DD, WD, CH, NT>), grid, block, 0, stream, p)
+#define NVA_ROPE_D(DD)                                     \
+  do {                                                     \
+    if (!wide && small) NVA_ROPE(DD, false, 1, false);       \
+    else if (!wide) NVA_ROPE(DD, false, kChunks, false);   \
+    else if (small) NVA_ROPE(DD, true, 1, false);          \
+    else NVA_ROPE(DD, true, kChunks, true);                \
+  } while (0)
+  if (p.head_dim == 128) NVA_ROPE_D(128);
+  else NVA_ROPE_D(64);
+#undef NVA_ROPE_D
+#undef NVA_ROPE
   return hipGetLastError();
 }
 

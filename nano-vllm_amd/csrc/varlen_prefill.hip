@@ -1142,7 +1142,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 //   23.6, 6 of 700-1400 27.0 -> 34.7; even above 12 tiles, 5 of 1024 22.4 -> 26.7, one of 8000
 //   127 -> 163.
 //   Up to 1024 cells: 24 of 300-700 36.0 -> 28.2, 8 of 2000 86.4 -> 73.0, one of 10000 252 -> 222, 32
-//   of 400 after 1024 cached 87.5 -> 75.8; uneven in 8 pairs, 4 of 500-4600 100 -> 128 (rotated 94),
+//   of 400 after 1024 cached 87.5 -> 75.8; uneven in 8 pairs, 4 of 500-4600 100 -> 128 (rotated 96),
 //   16 of 100-700 after 2048 cached 97 -> 112.
 //   1344 cells, 24 prompts: 35 -> 42.
 template <int KV, int D, bool STORE, bool PAIRED = false>

@@ -158,6 +158,32 @@ def test_head_chunks_and_narrow_rows(dev, nh, nkv, d, norm):
     assert torch.equal(q2.view(-1), q.view(-1)) and torch.equal(k2.view(-1), k.view(-1))
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(32, 8, 128), (4, 1, 128), (14, 2, 64)])
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_small_and_large_launches_agree(dev, nh, nkv, d, norm, aligned):
+    """The last size of the small launches (16384 head rows) and the first above it: the same rows
+    bit for bit, with 16-byte aligned rows and without."""
+    from nanovllm_amd import workloads as W
+    from nanovllm_amd.layers.qk_norm_rope import qk_norm_rope
+    T = 16384 // (nh + nkv)
+    c = W.make_producer_case(T + 1, nh, nkv, head_dim=d, norm=norm, seed=nh, device=dev)
+    q, k = c.q, c.k
+    if not aligned:
+        q = torch.empty(q.numel() + 4, dtype=q.dtype, device=dev)[4:].view(q.shape).copy_(q)
+
+    def run(n):
+        return qk_norm_rope(c.positions[:n].contiguous(), q[:n], k[:n], c.cos_sin_cache, nh, nkv, d, c.q_norm_weight,
+                            c.k_norm_weight, c.eps)
+    (ql, kl), (qs, ks) = run(T + 1), run(T)
+    torch.cuda.synchronize()
+    assert torch.equal(ql[:T], qs) and torch.equal(kl[:T], ks)
+    q1, k1 = (x.clone() for x in (q[T:], k[T:]))  # and the last token alone
+    q1, k1 = qk_norm_rope(c.positions[T:].contiguous(), q1, k1, c.cos_sin_cache, nh, nkv, d, c.q_norm_weight,
+                          c.k_norm_weight, c.eps)
+    assert torch.equal(ql[T:], q1) and torch.equal(kl[T:], k1)
+
+
 def test_out_of_range_positions_are_clamped(dev):
     from nanovllm_amd import workloads as W
     case = W.make_producer_case(3, 16, 8, max_position=64, positions=[-5, 64, 1000], seed=4, device=dev)
