@@ -95,7 +95,9 @@ struct PrefillParams {
   // key tiles (0: off) run as two workgroups over the two halves of their key
   // tiles, merged by the second to arrive.  At most split_slots such items;
   // each has kPrefillSplitCtlWords control words in split_ctl and
-  // kPrefillSplitPartFloats floats of partial results in split_part.
+  // kPrefillSplitPartFloats floats of partial results in split_part.  -1: off, and (two
+  // workgroups per CU) each query tile's (sequence, kv head) pairs start one XCD further on.
+  // (No field of its own: a longer argument block moved the other kernels' times by 0.5%.)
   int32_t split_tiles;
   int32_t split_slots;
   int32_t split_cus;          // compute units: with the real items, they cap the split items
@@ -118,7 +120,6 @@ struct PrefillParams {
   // bf16 paged kernel's scalar registers: 0.5% slower at 8813 tokens after 1024 cached.)
   const float* k_scale;
   const float* v_scale;
-  int32_t rotate;             // direct grid at d 64: a query tile's (sequence, kv head) pairs start one XCD on
 };
 
 struct QKNormRopeParams {

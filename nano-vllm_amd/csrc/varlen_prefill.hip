@@ -1134,7 +1134,7 @@ __device__ __forceinline__ void prefill_run(const PrefillParams& p, char* smem_a
 // for one, or with idle CUs key halves; above two, the persistent grid, which evens out
 // items of unequal work.  On this grid those stay uneven twice over: two heavy items on a
 // CU, and with a multiple of 8 (sequence, kv head) pairs the long sequences on their own
-// XCDs (p.rotate spreads their tiles over all, at the price of the L2 that they share).
+// XCDs (split_tiles -1 spreads their tiles over all, at the price of the L2 that they share).
 // Attention.forward, heads 14/2, unpaired (above 512 cells persistent) -> PAIRED, us.
 //   257 to 512 cells, short: 12 prompts of 100-1024 tokens 23.2 -> 18.9, 10 of 500 21.9 -> 17.8, 40
 //   of 200 after 256 cached 28.6 -> 27.0; uneven with at most 9/8 CUs' real items, 4 of 253-2022
@@ -1166,7 +1166,7 @@ __global__ __launch_bounds__(64 * kWaves, PAIRED ? 4 : 2) void varlen_prefill_ke
   } else {
     int x = blockIdx.x;
     if constexpr (PAIRED) {
-      if (p.rotate) x = static_cast<int>((blockIdx.x + blockIdx.y) % gridDim.x);
+      if (p.split_tiles < 0) x = static_cast<int>((blockIdx.x + blockIdx.y) % gridDim.x);
     }
     s = x / p.num_kv_heads;
     kvh = x - s * p.num_kv_heads;
@@ -1477,7 +1477,7 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
   const bool counted = store != nullptr && !p.block_table;
   const int64_t tokens = counted ? store->num_tokens : 0;
   const bool even = p.num_seqs == 1 || (counted && 20 * tokens >= 17 * int64_t{p.num_seqs} * max_seqlen_q);
-  bool paired = false;
+  bool paired = false, rotate = false;
   if (p.head_dim == 64 && max_items > cus && max_items <= 2 * int64_t{cus}) {
     // real items, a half tile more per sequence than the rows fill
     const int64_t real = p.num_kv_heads * tokens / p.positions_per_tile + pairs / 2;
@@ -1485,7 +1485,7 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
              (counted && !even && 8 * real <= 9 * int64_t{cus});
   } else if (p.head_dim == 64 && max_items > cus && max_items <= 4 * int64_t{cus}) {
     paired = counted || even || pairs % kXcds != 0 || kt_max <= kPairedTilesTwo;
-    p.rotate = counted && !even && pairs % kXcds == 0;
+    rotate = counted && !even && pairs % kXcds == 0;
   }
   const bool persistent = p.num_seqs <= kPersistMaxSeqs && p.num_q_tiles <= kPersistMaxTiles &&
                           max_items > 2 * int64_t{cus} && !paired;
@@ -1534,7 +1534,7 @@ hipError_t launch_prefill(const PrefillParams& p0, int max_seqlen_q, int max_seq
 #undef NVA_PERSIST
     return hipGetLastError();
   }
-  p.split_tiles = 0;
+  p.split_tiles = rotate ? -1 : 0;
   p.split_slots = kPrefillSplitSlots;
   p.split_cus = cus;
   const int64_t pairs_split = kPrefillSplitSlots / p.num_kv_heads;  // at most this many pairs split
