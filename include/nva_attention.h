@@ -143,8 +143,9 @@ int nva_prefill_fp8(const void* q, int64_t q_row_stride,
  * over them (nva_prefill with block_table NULL), with the results of the two calls.  The
  * attention reads the fresh rows, not the caches, so over a bf16 cache with 16-byte aligned
  * rows the store runs inside the prefill launch; otherwise (an fp8 cache, other alignments,
- * GQA group 1 at head_dim 128, a large launch without a workspace, or q, k, v or out inside a
- * cache) the store kernel runs first.  num_queries: rows of q and out.
+ * GQA group 1 but in the small launches of half-row items, a large launch without a
+ * workspace, or q, k, v or out inside a cache) the store kernel runs first.  num_queries:
+ * rows of q and out.
  */
 int nva_store_prefill(void* k_cache, void* v_cache, int64_t num_slots,
                       const int32_t* slot_mapping, int64_t num_tokens, int32_t cache_dtype,
@@ -216,7 +217,7 @@ int nva_decode(const void* q, int64_t q_row_stride,
  * with no extra launch: for a sequence with keys, the wave that reads key cache_seqlens[b]-1
  * writes the new rows and uses them from registers; the rows of a sequence with none
  * (cache_seqlens[b] == 0, e.g. a padded graph row) are written by the merge kernel, after
- * every read of the call.  The result is deterministic for any input and equals
+ * every read of the call.  The result is deterministic for distinct valid slots and equals
  * store-then-decode when (a) slot_mapping[b] is the slot of key cache_seqlens[b]-1 for every
  * sequence with keys, as every decode step the reference runs has it (prepare_decode,
  * model_runner.py:218-229), and (b) no sequence reads the slot of a row with no keys.  The

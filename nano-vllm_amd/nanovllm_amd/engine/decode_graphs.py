@@ -15,12 +15,13 @@ static inputs (in the model they come from the layer's projection).
 
 Padding of the slot mapping (reference quirk Q1).  The reference zero-fills it,
 so padded rows write their K/V into slot 0, which may belong to a live sequence.
-pad_slot=0 reproduces that exactly: each layer runs the reference's two calls
-(store, then decode), so a live sequence owning slot 0 reads the padded row as
-the reference's does.  The default pad_slot=-1 is skipped by the store: padded
-rows leave the cache alone and produce zero rows, and with no padded row writing
-a slot, each layer's store runs inside its decode launch (Attention's
-fuse_decode_store), one graph node fewer per layer.
+pad_slot=0 reproduces that exactly: each layer has the results of the reference's two
+calls, store then decode (nva_store_then_decode: one launch and a merge for small
+batches, two launches and a merge above), so a live sequence owning slot 0 reads the
+padded row as the reference's does.  The default pad_slot=-1 is skipped by the store:
+padded rows leave the cache alone and produce zero rows, and with no padded row writing
+a slot, each layer's store runs inside its decode launch at any batch (Attention's
+fuse_decode_store).
 """
 from __future__ import annotations
 

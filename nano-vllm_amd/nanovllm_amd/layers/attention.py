@@ -389,7 +389,10 @@ class Attention(nn.Module):
 
     fuse_decode_store (not in the reference, default False): when True the decode
     branch runs the store and the attention as one call (store_and_decode), one
-    launch fewer per layer.  It equals the reference's store-then-decode only if no
+    launch fewer per layer in the balanced mode; small batches store inside the decode
+    launch by default too (nva_store_then_decode), and with tables of at most eight 32-key
+    steps the default is the shorter form, a single launch.  It equals the reference's
+    store-then-decode only if no
     padded row (context length 0) carries a slot that a live sequence reads; the
     reference's run_model zero-fills slot_mapping (model_runner.py:271-273), so its
     padded rows write slot 0 of block 0, which a live sequence may own.  Set it only
